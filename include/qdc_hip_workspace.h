@@ -1,0 +1,37 @@
+/* qdc_hip_workspace.h -- entry points of libqdc_hip.so that work through a
+ * caller's scratch buffer or replace several entry points of qdc_hip.h by one
+ * pass.  Types, status codes, dtype codes and stream rules are those of
+ * qdc_hip.h: nothing is allocated or kept, everything is enqueued on `stream`,
+ * and a negative status is returned before anything is enqueued.
+ */
+#ifndef QDC_HIP_WORKSPACE_H
+#define QDC_HIP_WORKSPACE_H
+
+#include "qdc_hip.h"
+
+#ifdef __cplusplus
+extern "C" {
+#endif
+
+/* Bytes of 16-byte aligned device scratch that qdc_delta_scan_ws needs for these
+ * sizes, or 0 when it has no form for them (call qdc_delta_scan then): key_dim
+ * 32, 64 or 128 and value_dim a multiple of 16. */
+int64_t qdc_delta_scan_workspace(int64_t batch, int64_t seq, int64_t heads, int64_t key_dim,
+                                 int64_t value_dim);
+
+/* The recurrence of qdc_delta_scan, the same arguments and results, as two
+ * launches: what does not involve the state is computed for all chunks of 16
+ * tokens at once into `workspace` (workspace_bytes >= qdc_delta_scan_workspace),
+ * then the state runs over the chunks.  q, k and v must be 16-byte aligned with
+ * ld_qk and ld_v multiples of 4 below 2^25 (QDC_ERR_SHAPE otherwise); the workspace may not
+ * overlap any other argument. */
+int32_t qdc_delta_scan_ws(void *out, int32_t out_dtype, const float *q, const float *k,
+                          const float *v, const float *beta, const float *decay, int64_t batch,
+                          int64_t seq, int64_t heads, int64_t key_heads, int64_t key_dim,
+                          int64_t value_dim, int64_t ld_qk, int64_t ld_v, void *workspace,
+                          int64_t workspace_bytes, hipStream_t stream);
+
+#ifdef __cplusplus
+}
+#endif
+#endif

@@ -65,6 +65,13 @@ SIGNATURES = {
     "qdc_row_scale_check": (_i32, [ctypes.c_uint32, _i64, _vp, _vp]),
 }
 
+# the entry points of include/qdc_hip_workspace.h, likewise
+WORKSPACE_SIGNATURES = {
+    "qdc_delta_scan_workspace": (_i64, [_i64] * 5),
+    "qdc_delta_scan_ws": (_i32, [_vp, _i32, _vp, _vp, _vp, _vp, _vp] + [_i64] * 8
+                          + [_vp, _i64, _vp]),
+}
+
 _lib = None
 
 
@@ -81,7 +88,7 @@ def lib():
                 f"{LIB_PATH} is not built; run `make -C qwendecisioncore.jl_amd/csrc` "
                 "or __graft_entry__.build()")
         handle = ctypes.CDLL(LIB_PATH)
-        for name, (res, args) in SIGNATURES.items():
+        for name, (res, args) in (SIGNATURES | WORKSPACE_SIGNATURES).items():
             fn = getattr(handle, name)
             fn.restype = res
             fn.argtypes = args

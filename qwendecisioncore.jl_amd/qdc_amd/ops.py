@@ -606,10 +606,23 @@ def delta_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, beta: torch.Te
     _device(q, out)
     if out.shape != (B, S, H, vd) or out.dtype not in _DTYPES or not out.is_contiguous():
         raise ValueError("out must be a contiguous [B, S, H, vd] float32/bfloat16 tensor")
-    out_dtype = out.dtype
-    check(lib().qdc_delta_scan(out.data_ptr(), _DTYPES[out_dtype], q.data_ptr(), k.data_ptr(),
-                               v.data_ptr(), beta.data_ptr(), decay.data_ptr(), B, S, H, KH, kd,
-                               vd, ld_k, ld_v, _stream(q)), "delta_scan")
+    args = (out.data_ptr(), _DTYPES[out.dtype], q.data_ptr(), k.data_ptr(), v.data_ptr(),
+            beta.data_ptr(), decay.data_ptr(), B, S, H, KH, kd, vd, ld_k, ld_v)
+    # The two-launch form wherever it takes the sizes and the 16-byte rows, but for
+    # sequences of so few chunks of 16 tokens that its second launch is not earned
+    # back (kd = vd = 128, two launches / one, microseconds: 16 tokens, 4 heads
+    # 8.2 / 6.3; 32 tokens, 4 heads 9.3 / 9.6; 33 tokens, 16 heads 10.2 / 12.7; from
+    # 513 slices of 16 value columns on, 8 sequences of 33 tokens 14.7 / 13.7, of 64
+    # tokens 17.3 / 17.6).
+    long = S > (48 if B * H * (vd // 16) > 512 else 32)
+    rows16 = (ld_k % 4 == 0 and ld_v % 4 == 0 and max(ld_k, ld_v) < 1 << 25
+              and not any(t.data_ptr() % 16 for t in (q, k, v)))
+    need = lib().qdc_delta_scan_workspace(B, S, H, kd, vd) if long and rows16 else 0
+    if need:
+        work = torch.empty(need, dtype=torch.uint8, device=q.device)
+        check(lib().qdc_delta_scan_ws(*args, work.data_ptr(), need, _stream(q)), "delta_scan")
+    else:
+        check(lib().qdc_delta_scan(*args, _stream(q)), "delta_scan")
     return out
 
 

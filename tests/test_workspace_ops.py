@@ -1,0 +1,107 @@
+"""The entry points of include/qdc_hip_workspace.h: the recurrence through a
+workspace, at the edges of its chunks, slices and wavefront splits, against the
+token-by-token oracle; and its argument checks, which need no GPU."""
+import os
+import re
+
+import numpy as np
+import pytest
+import torch
+
+from conftest import ROOT, normwise
+from qdc_amd import _lib
+
+F32, BF16, X2 = _lib.QDC_F32, _lib.QDC_BF16, _lib.QDC_BF16X2
+FAKE = 0x10000  # a non-null, 16-byte aligned address never dereferenced by validation
+BIG = 1 << 60
+
+
+def test_exports_match_header():
+    text = open(os.path.join(ROOT, "include", "qdc_hip_workspace.h")).read()
+    names = set(re.findall(r"^\s*\w+\s+(qdc_\w+)\s*\(", text, re.M))
+    assert names == set(_lib.WORKSPACE_SIGNATURES)
+    for name in names:
+        assert hasattr(_lib.lib(), name), name
+
+
+def test_delta_scan_ws_validation():
+    lib = _lib.lib()
+    size = lib.qdc_delta_scan_workspace
+    need = size(2, 33, 4, 128, 48)
+    assert need == 2 * 4 * 3 * 544 * 4
+    assert size(2, 33, 4, 96, 48) == 0 and size(2, 33, 4, 256, 48) == 0  # key_dim
+    assert size(2, 33, 4, 128, 40) == 0                                  # value_dim % 16
+    assert size(0, 33, 4, 128, 48) == 0 and size(2, 0, 4, 128, 48) == 0
+    assert size(1, 1 << 30, 4, 128, 48) == 0                             # too many chunks
+
+    def f(out=FAKE, dt=F32, q=FAKE, k=FAKE, v=FAKE, beta=FAKE, decay=FAKE, batch=2, seq=33,
+          heads=4, kh=2, kd=128, vd=48, ld_qk=256, ld_v=192, ws=FAKE + (1 << 30), nbytes=need):
+        return lib.qdc_delta_scan_ws(out, dt, q, k, v, beta, decay, batch, seq, heads, kh, kd, vd,
+                                     ld_qk, ld_v, ws, nbytes, None)
+
+    assert f(dt=7) == -3
+    assert f(heads=3) == -2 and f(kd=96) == -2 and f(vd=40) == -2
+    assert f(ld_qk=255) == -2 and f(ld_v=191) == -2 and f(ld_qk=258) == -2
+    assert f(nbytes=need - 1) == -2
+    assert f(q=FAKE + 4) == -2 and f(ws=FAKE + (1 << 30) + 8) == -2
+    for name in ("out", "q", "k", "v", "beta", "decay", "ws"):
+        assert f(**{name: None}) == -1, name
+    for name in ("out", "q", "k", "v", "beta", "decay"):  # workspace over another argument
+        assert f(**{name: FAKE + (1 << 30) + 16}) == -5, name
+    assert f(seq=0, out=None) == 0 and f(batch=0, out=None) == 0
+
+
+# key_dim x value_dim; heads and batch on both sides of 512 slices of 16 columns
+# (whole slices / key parts), value_dim leaving 1..4 slices in the last workgroup
+SCAN = [(1, 1, 1, 1, 128, 16), (1, 15, 1, 2, 128, 48), (2, 16, 2, 2, 64, 32), (1, 17, 2, 4, 32, 80),
+        (1, 33, 1, 1, 32, 16), (2, 49, 1, 2, 128, 128), (9, 33, 4, 64, 128, 16),
+        (6, 17, 16, 32, 128, 48), (5, 31, 8, 32, 64, 64), (3, 48, 8, 64, 32, 80),
+        (4, 1, 16, 64, 128, 48), (4, 32, 64, 64, 128, 32)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,S,KH,H,kd,vd", SCAN)
+def test_delta_scan_ws_edges(B, S, KH, H, kd, vd):
+    """fp32 sums of at most 3 kd products a token, errors of about 1e-7 as in the
+    other forms: the repository's fp32 bar of 1e-5 per sequence, and every element
+    within 1e-5 of the largest output of its sequence."""
+    from oracle import forward
+    from qdc_amd import ops
+    rng = np.random.default_rng(S * 1000 + kd + vd)
+    q = rng.standard_normal((B, S, KH, kd), dtype=np.float32)
+    k = rng.standard_normal((B, S, KH, kd), dtype=np.float32)
+    q /= np.linalg.norm(q, axis=-1, keepdims=True) * np.float32(np.sqrt(kd))
+    k /= np.linalg.norm(k, axis=-1, keepdims=True)
+    v = rng.standard_normal((B, S, H, vd), dtype=np.float32)
+    beta = rng.random((B, S, H), dtype=np.float32)
+    decay = -rng.random((B, S, H), dtype=np.float32) * np.float32(0.5)
+    # the column blocks of rows with other data around them
+    rows = torch.full((B, S, 2 * KH * kd + H * vd + 8), float("nan"), device="cuda")
+    views = []
+    at = 4
+    for x in (q, k, v):
+        w = x.shape[2] * x.shape[3]
+        rows[..., at:at + w] = torch.from_numpy(x.reshape(B, S, w)).cuda()
+        views.append(rows[..., at:at + w].unflatten(-1, x.shape[2:]))
+        at += w
+    gates = [torch.from_numpy(x).cuda() for x in (beta, decay)]
+    lib = _lib.lib()
+    need = lib.qdc_delta_scan_workspace(B, S, H, kd, vd)
+    assert need > 0
+    out = {}
+    for dtype, code in ((torch.float32, F32), (torch.bfloat16, BF16)):
+        work = torch.full((need // 4,), float("nan"), device="cuda")  # all of it is written first
+        out[dtype] = torch.empty((B, S, H, vd), dtype=dtype, device="cuda")
+        ld = rows.shape[-1]
+        _lib.check(lib.qdc_delta_scan_ws(out[dtype].data_ptr(), code,
+                                         *(t.data_ptr() for t in views + gates), B, S, H, KH, kd,
+                                         vd, ld, ld, work.data_ptr(), need,
+                                         torch.cuda.current_stream().cuda_stream), "scan")
+    assert torch.equal(out[torch.bfloat16], out[torch.float32].bfloat16())
+    got = out[torch.float32].cpu().numpy()
+    if S > 48:  # the operator takes this form
+        assert torch.equal(ops.delta_scan(*views, *gates), out[torch.float32])
+    for b in range(B):
+        exp = forward.delta_recurrence(q[b], k[b], v[b], beta[b], decay[b])
+        assert normwise(got[b], exp) <= 1e-5
+        assert np.abs(got[b] - exp).max() <= 1e-5 * np.abs(exp).max()
