@@ -31,6 +31,24 @@ int32_t qdc_delta_scan_ws(void *out, int32_t out_dtype, const float *q, const fl
                           int64_t value_dim, int64_t ld_qk, int64_t ld_v, void *workspace,
                           int64_t workspace_bytes, hipStream_t stream);
 
+/* Causal attention of prepared (normalised, rotated) heads with its output gate:
+ *     out[t, h*head_dim + r] = sigmoid(gate[t, h, r]) *
+ *         sum_j softmax_j(scale * q[t, h] . k[j, g]) v[j, g, r],  g = h / (heads/kv_heads)
+ * over the keys j of the same sequence with j <= t whose mask[b, j] != 0 (mask
+ * null: all); a query that sees no key weighs every key of its sequence alike.
+ * What qdc_attention_softmax and qdc_attention_gate give around two batched
+ * products, with no score matrix.  `dtype` is the type of q, k, v and gate, which
+ * are views of rows of head_dim contiguous elements with their strides between
+ * tokens and heads in elements; out_dtype may also be QDC_BF16X2.  head_dim 64,
+ * 128 or 256; all strides multiples of 16 bytes and all pointers 16-byte aligned
+ * (QDC_ERR_SHAPE otherwise).  out may not overlap any input. */
+int32_t qdc_attention_fused(void *out, int32_t out_dtype, const void *q, const void *k,
+                            const void *v, const void *gate, const int32_t *mask, int64_t batch,
+                            int64_t seq, int64_t heads, int64_t kv_heads, int64_t head_dim,
+                            int64_t q_tok, int64_t q_head, int64_t k_tok, int64_t k_head,
+                            int64_t v_tok, int64_t v_head, int64_t gate_tok, int64_t gate_head,
+                            int64_t out_tok, float scale, int32_t dtype, hipStream_t stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -70,6 +70,8 @@ WORKSPACE_SIGNATURES = {
     "qdc_delta_scan_workspace": (_i64, [_i64] * 5),
     "qdc_delta_scan_ws": (_i32, [_vp, _i32, _vp, _vp, _vp, _vp, _vp] + [_i64] * 8
                           + [_vp, _i64, _vp]),
+    "qdc_attention_fused": (_i32, [_vp, _i32, _vp, _vp, _vp, _vp, _vp] + [_i64] * 14
+                            + [_f32, _i32, _vp]),
 }
 
 _lib = None

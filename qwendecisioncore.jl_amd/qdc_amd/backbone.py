@@ -19,14 +19,15 @@ later layer's input RMSNorm with the previous layer's MLP
 residual add (``qdc_residual_rmsnorm``; the last one with the final norm) and,
 before a DeltaNet layer, with its input mask (``qdc_residual_rmsnorm_masked``),
 post-attention residual + RMSNorm, the attention prologue (q/k norm + partial
-RoPE, and K transposed and V head-major for the two products, read straight out
-of the packed projection), the attention masked softmax and output-gate merge, the
-DeltaNet prologue (convolution, SiLU, q/k L2 norm, gates), the gated-delta
+RoPE, read straight out of the packed projection), causal attention with its
+masked softmax and output gate in one pass over the heads, the DeltaNet prologue (convolution, SiLU, q/k L2 norm, gates), the gated-delta
 recurrence, the DeltaNet gated RMSNorm reading z inside the packed projection,
-and SwiGLU reading the packed gate||up GEMM output.  GEMMs and the two attention
-products run through PyTorch-ROCm (hipBLASLt), with fp32 results; attention
-scores and probabilities are fp32 (probabilities stored in the model dtype for
-the PV product).
+and SwiGLU reading the packed gate||up GEMM output.  GEMMs run through
+PyTorch-ROCm (hipBLASLt), with fp32 results; attention scores, exponentials and
+their sums are fp32 (the exponentials enter the product with V in the model
+dtype).  Head sizes the attention kernel does not take, and the last-token
+forward's single query per head, run the two attention products as batched GEMMs
+around the softmax and gate kernels.
 
 ``split_gemm_inputs=True`` (or ``"all"``; bf16 models) stores every GEMM input
 -- the normalised rows, the SwiGLU output, the merged attention output and the
@@ -254,13 +255,14 @@ class QwenBackbone:
 
     def _full_attention(self, layer, x, mask32, B, S):
         """``full_attention`` in the AMDGPU form (``ext/amdgpu_attention.jl:108-178``;
-        generic ``src/backbone.jl:224-262``).  One prologue launch normalises and
-        rotates q and k and moves v out of the packed projection into the layouts
-        the products read: q ``[B, H, S, hd]``, K transposed ``[B, KV, hd, S]``,
-        v ``[B, KV, S, hd]``.  The G = H / KV query heads sharing a KV head are one
-        ``[G*S, hd]`` block, so both products are plain batched GEMMs over
-        (sequence, KV head), with no K/V expansion and no layout copy.  The
-        masked softmax and the gate merge are HIP kernels."""
+        generic ``src/backbone.jl:224-262``): q and k normalised and rotated out of
+        the packed projection, then scores, masked softmax, the product with v and
+        the output gate in one kernel that reads v and the gate inside the
+        projection.  Other head sizes: one prologue launch writes q
+        ``[B, H, S, hd]``, K transposed ``[B, KV, hd, S]`` and v ``[B, KV, S, hd]``, so
+        that with the G = H / KV query heads of a KV head as one ``[G*S, hd]`` block
+        both products are plain batched GEMMs, around the softmax and gate
+        kernels."""
         cfg = self.cfg
         hd, H, KV = cfg.head_dim, cfg.heads, cfg.kv_heads
         G = H // KV
@@ -271,10 +273,16 @@ class QwenBackbone:
         v_in = proj[:, (H + KV) * hd:(H + 2 * KV) * hd].view(T, KV, hd)
         gate = proj[:, (H + 2 * KV) * hd:].view(T, H, hd)
         tables = self.rope_tables(S) if cfg.rotary_dim else None
+        scale = float(np.float32(1) / np.sqrt(np.float32(hd)))      # inv(sqrt(Float32(dim)))
+        if ops.attention_fused_takes(self.dtype, hd):
+            q, k = ops.prepare_heads(q_in, k_in, layer["q_norm"], layer["k_norm"], tables,
+                                     cfg.rotary_dim, cfg.eps, seq_len=S)
+            merged = ops.attention_fused(q, k, v_in, gate, mask32, scale, B,
+                                         out_dtype=self.gemm_in or self.dtype)
+            return self._mm32(merged, layer["out"])
         q, kt, v = ops.attention_prepare(q_in, k_in, v_in, layer["q_norm"], layer["k_norm"],
                                          tables, cfg.rotary_dim, cfg.eps, B)
         scores = self._bmm32(q.view(B * KV, G * S, hd), kt.view(B * KV, hd, S))  # [B*KV, G*S, S]
-        scale = float(np.float32(1) / np.sqrt(np.float32(hd)))      # inv(sqrt(Float32(dim)))
         probs = ops.attention_softmax(scores.view(B, H, S, S), mask32, scale, out_dtype=self.dtype,
                                       out=scores.view(B, H, S, S) if self.dtype == torch.float32
                                       else None)

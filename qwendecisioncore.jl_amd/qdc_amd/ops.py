@@ -747,6 +747,51 @@ def attention_gate(values: torch.Tensor, gate: torch.Tensor, out_dtype=None,
     return out
 
 
+def attention_fused_takes(dtype: torch.dtype, head_dim: int) -> bool:
+    """Whether :func:`attention_fused` has a kernel for these heads."""
+    return dtype in _DTYPES and head_dim in (64, 128, 256)
+
+
+def attention_fused(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, gate: torch.Tensor,
+                    mask: torch.Tensor | None, scale: float, batch: int,
+                    out_dtype=None) -> torch.Tensor:
+    """Causal attention and its output gate in one pass over prepared heads: what
+    :func:`attention_softmax` and :func:`attention_gate` give around two batched
+    products, without the score matrix.  ``q`` and ``gate`` ``[T, H, hd]``, ``k``
+    and ``v`` ``[T, KV, hd]`` (views with contiguous rows) of ``batch`` sequences of
+    ``T // batch`` tokens, ``mask`` int32 ``[batch, T // batch]`` or None ->
+    ``[T, H*hd]`` in ``out_dtype`` (default: q's dtype; ``BF16X2`` writes
+    ``[T, 2*H*hd]``)."""
+    _device(q, k, v, gate)
+    code = _dtype_code(q, k, v, gate)
+    if q.dim() != 3 or k.dim() != 3 or gate.shape != q.shape or v.shape != k.shape:
+        raise ValueError("q and gate must be [T, H, hd], k and v [T, KV, hd]")
+    T, H, hd = q.shape
+    KV = k.shape[1]
+    if k.shape[0] != T or k.shape[2] != hd or batch <= 0 or T % batch or KV == 0 or H % KV:
+        raise ValueError("q, k and v must share tokens and head_dim; tokens a multiple of batch")
+    S = T // batch
+    for t in (q, k, v, gate):
+        if t.stride(2) != 1:
+            raise ValueError("rows must be contiguous")
+    if mask is not None:
+        _device(q, mask)
+        if mask.dtype != torch.int32 or mask.shape != (batch, S) or not mask.is_contiguous():
+            raise ValueError("mask must be a contiguous int32 [batch, T // batch] tensor")
+    split = _is_split(out_dtype)
+    odt = torch.bfloat16 if split else out_dtype or q.dtype
+    out = torch.empty((T, 2 * H * hd if split else H * hd), dtype=odt, device=q.device)
+    tok = lambda t: t.stride(0) if T > 1 else t.shape[1] * hd  # noqa: E731
+    head = lambda t: t.stride(1) if t.shape[1] > 1 else hd  # noqa: E731
+    strides = [f(t) for t in (q, k, v, gate) for f in (tok, head)]
+    check(lib().qdc_attention_fused(out.data_ptr(), _lib.QDC_BF16X2 if split else _DTYPES[odt],
+                                    q.data_ptr(), k.data_ptr(), v.data_ptr(), gate.data_ptr(),
+                                    0 if mask is None else mask.data_ptr(), batch, S, H, KV, hd,
+                                    *strides, H * hd, scale, code, _stream(q)),
+          "attention_fused")
+    return out
+
+
 def device_copy(dst: torch.Tensor, src: torch.Tensor, chunks_per_thread: int = 1,
                 block: int = 256) -> torch.Tensor:
     """Plain copy of ``src``'s bytes into ``dst`` (both contiguous, same byte

@@ -105,3 +105,81 @@ def test_delta_scan_ws_edges(B, S, KH, H, kd, vd):
         exp = forward.delta_recurrence(q[b], k[b], v[b], beta[b], decay[b])
         assert normwise(got[b], exp) <= 1e-5
         assert np.abs(got[b] - exp).max() <= 1e-5 * np.abs(exp).max()
+
+
+def test_attention_fused_validation():
+    lib = _lib.lib()
+
+    def f(out=FAKE, odt=BF16, q=BIG, k=BIG, v=BIG, gate=BIG, mask=None, batch=2, seq=33, heads=4,
+          kv=2, hd=64, q_tok=256, q_head=64, k_tok=128, k_head=64, v_tok=128, v_head=64,
+          g_tok=256, g_head=64, o_tok=256, dt=BF16):
+        return lib.qdc_attention_fused(out, odt, q, k, v, gate, mask, batch, seq, heads, kv, hd,
+                                       q_tok, q_head, k_tok, k_head, v_tok, v_head, g_tok, g_head,
+                                       o_tok, 0.125, dt, None)
+
+    assert f(odt=7) == -3 and f(dt=X2) == -3
+    assert f(heads=3) == -2 and f(hd=96) == -2 and f(kv=0) == -2 and f(batch=-1) == -2
+    assert f(q_tok=260) == -2 and f(k_head=68) == -2 and f(v_tok=130) == -2  # 16-byte rows
+    assert f(v_head=32) == -2 and f(g_tok=260) == -2 and f(g_head=68) == -2
+    assert f(o_tok=248) == -2 and f(o_tok=260) == -2
+    assert f(q=BIG + 8) == -2 and f(out=FAKE + 4) == -2 and f(mask=BIG + 2) == -2
+    for name in ("out", "q", "k", "v", "gate"):
+        assert f(**{name: None}) == -1, name
+    for name in ("q", "k", "v", "gate", "mask"):
+        assert f(**{name: FAKE + 16}) == -5, name
+    assert f(seq=0, out=None) == 0 and f(batch=0, out=None) == 0
+
+
+# lengths around the tiles of 32 queries and keys; 1..6 query heads per KV head, so
+# that a workgroup's four units cross query blocks; every head size
+ATTENTION = [(1, 1, 2, 1, 64, "none"), (2, 31, 6, 6, 64, "holes"), (1, 32, 3, 1, 128, "prefix"),
+             (3, 33, 5, 1, 128, "holes"), (2, 65, 8, 2, 256, "prefix"), (1, 97, 6, 1, 256, "none"),
+             (1, 160, 4, 2, 64, "none"), (2, 64, 2, 2, 256, "first"), (1, 200, 4, 1, 128, "first")]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("out", ["f32", "bf16", "split"])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("B,S,H,KV,hd,kind", ATTENTION)
+def test_attention_fused_edges(B, S, H, KV, hd, kind, dtype, out):
+    """Against 64 bits on the same inputs.  Per element the bf16 form may differ by
+    the rounding of the weights, 2^-8 of the weighted mean of |v| (each weight is
+    rounded by at most 2^-9 and so is what it replaces), the fp32 form by fp32 sums
+    (1e-5 of it); then by the rounding of the output (bf16 2^-9, two terms 2^-17)."""
+    from qdc_amd import ops
+    rng = np.random.default_rng(S * 10 + H + hd)
+    T = B * S
+    # q | k | v | gate as the packed projection holds them, scores of a few units
+    proj = torch.from_numpy(rng.standard_normal((T, (2 * H + 2 * KV) * hd), dtype=np.float32))
+    proj[:, :H * hd] *= 2.0
+    proj = proj.to(dtype).cuda()
+    q, k, v, gate = (x.unflatten(1, (-1, hd)) for x in
+                     proj.split([H * hd, KV * hd, KV * hd, H * hd], 1))
+    mask = None
+    if kind != "none":
+        m = np.ones((B, S), np.int32)
+        if kind == "prefix":       # the first queries see no key: an even spread over all
+            m[:, :S // 2] = 0
+        elif kind == "first":      # nothing kept but the last key
+            m[:, :-1] = 0
+        else:
+            m[rng.random((B, S)) < 0.4] = 0
+        mask = torch.from_numpy(m)
+    scale = hd ** -0.5
+    got = ops.attention_fused(q, k, v, gate, None if mask is None else mask.cuda(), scale, B,
+                              out_dtype={"f32": torch.float32, "bf16": torch.bfloat16,
+                                         "split": ops.BF16X2}[out])
+    got = (ops.join_split(got) if out == "split" else got).double().cpu().view(B, S, H, hd)
+    assert torch.isfinite(got).all()
+    q, k, v, gate = (x.cpu().double().view(B, S, -1, hd).transpose(1, 2) for x in (q, k, v, gate))
+    k, v = (x.repeat_interleave(H // KV, 1) for x in (k, v))
+    see = torch.ones(S, S, dtype=torch.bool).tril()[None, None]
+    if mask is not None:
+        see = see & mask.bool()[:, None, None, :]
+    low = -torch.finfo(torch.float32).max
+    p = torch.softmax((q @ k.transpose(2, 3) * scale).masked_fill(~see, low), -1)
+    exact = (torch.sigmoid(gate) * (p @ v)).transpose(1, 2)
+    spread = (torch.sigmoid(gate) * (p @ v.abs())).transpose(1, 2)
+    bound = spread * (1e-5 if dtype == torch.float32 else 2.0 ** -8 + 1e-5)
+    bound = bound + exact.abs() * {"f32": 0.0, "bf16": 2.0 ** -8, "split": 2.0 ** -16}[out] + 1e-30
+    assert ((got - exact).abs() <= bound).all(), ((got - exact).abs() / bound).max()
