@@ -22,9 +22,10 @@
 // it when the slices fill the chip, the chain from one chunk's state to the next
 // when they do not.  Both launches, kd = vd = 128, against the one-launch form of
 // qdc_delta_scan.hip, which runs 64 columns in eight wavefronts that meet twice a
-// chunk: 8 x 2048 tokens, 16 heads 326 us (prepare 56) / 420; the same with 32 heads
-// 578 / 833; 2 x 1501, 32 heads 182 / 307; 1 x 777, 16 heads 57 / 161; 1 x 411, 4 heads
-// 32 / 86.  Without the operands' refills (timing only) the scan of 8 x 2048 tokens
+// chunk: 8 x 2048 tokens, 16 heads 319 us (prepare 56) / 420; the same with 32 heads
+// 547 / 836; 2 x 1501, 32 heads 169 / 307; 1 x 777, 16 heads 55 / 161; 1 x 411, 4 heads
+// 32 / 87.  Running addresses of rows and outputs as uniform bases and lane offsets
+// are 27 and 39 us of the first two.  Without the operands' refills (timing only) the scan of 8 x 2048 tokens
 // takes 227 us, so what its loads cost beside the products is the next thing to gain.
 #include "qdc_common.hpp"
 #include "qdc_hip_workspace.h"
@@ -244,8 +245,13 @@ __global__ __launch_bounds__(KSPLIT > 1 ? KSPLIT * kWave : kBlock, 2) void delta
     const int h = (int)(bh - b * a.by_heads.d), g = h / a.groups;
     const int S = a.S, chunks = a.chunks;
     const int64_t row0 = (int64_t)b * S, o_tok = (int64_t)a.H * a.vd;
-    TO *ob = reinterpret_cast<TO *>(a.out) + row0 * o_tok + (int64_t)h * a.vd + col +
-             4 * lg * o_tok;
+    // where the output rows of the chunk to be stored start (uniform)
+    TO *oc = reinterpret_cast<TO *>(a.out) + row0 * o_tok + (int64_t)h * a.vd;
+    uint32_t off_o[PARTS];  // this lane's byte offsets from there
+#pragma unroll
+    for (int j = 0; j < PARTS; ++j)
+        off_o[j] = (uint32_t)sizeof(TO) *
+                   ((uint32_t)(4 * lg + ks * PARTS + j) * (uint32_t)o_tok + (uint32_t)col);
 
     // where the operands of the chunk being fetched start (uniform), and this
     // lane's byte offsets from there; in the last chunk, tokens past the end read
@@ -279,14 +285,26 @@ __global__ __launch_bounds__(KSPLIT > 1 ? KSPLIT * kWave : kBlock, 2) void delta
     };
     // SHARED: chunk c's rows to registers, and from there to its tile
     f32x4 stage[2][PIECES];
-    auto load_rows = [&](int c) {
-        const int t0 = min(c, chunks - 1) * kC;  // past the end: not used
+    const float *kr = kc, *qr = qc;  // rows of the chunk to be loaded (uniform)
+    uint32_t off_r[PIECES];          // this thread's byte offsets from there
+    auto row_offsets = [&](int top) {
 #pragma unroll
         for (int p = 0; p < PIECES; ++p) {
-            const int i = threadIdx.x + p * kBlock, r = min(i / (4 * KB), min(kC, S - t0) - 1);
-            const int64_t o = (int64_t)(t0 + r) * a.ld_qk + 4 * (i % (4 * KB));
-            stage[0][p] = load4(kc + o);
-            stage[1][p] = load4(qc + o);
+            const int i = threadIdx.x + p * kBlock;
+            off_r[p] = 4u * ((uint32_t)min(i / (4 * KB), top) * (uint32_t)a.ld_qk +
+                             4u * (i % (4 * KB)));
+        }
+    };
+    auto load_rows = [&](int c) {  // the chunks in order; past the end: not used
+        if (c + 1 == chunks) row_offsets(S - 1 - c * kC);
+#pragma unroll
+        for (int p = 0; p < PIECES; ++p) {
+            stage[0][p] = load4(at(kr, off_r[p]));
+            stage[1][p] = load4(at(qr, off_r[p]));
+        }
+        if (c + 1 < chunks) {
+            kr += kstep;
+            qr += kstep;
         }
     };
     auto write_rows = [&](int c) {
@@ -330,18 +348,20 @@ __global__ __launch_bounds__(KSPLIT > 1 ? KSPLIT * kWave : kBlock, 2) void delta
         x.eg = load4(at(rc + kRecEg, 16u * lg));
         x.et = load4(at(rc + kRecEt, 16u * lg));
     };
-    // this key part's rows of the output of chunk c
+    // this key part's rows of the output of chunk c, the chunks in order
     auto store = [&](int c, const float (&o)[PARTS]) {
+        char *dst = reinterpret_cast<char *>(oc);
+        oc += kC * o_tok;
         if (!live) return;
-        TO *dst = ob + (int64_t)(c * kC + ks * PARTS) * o_tok;
+        const int left = S - c * kC - 4 * lg - ks * PARTS;
         if ((c + 1) * kC <= S) {
 #pragma unroll
-            for (int j = 0; j < PARTS; ++j) dst[j * o_tok] = from_f32<TO>(o[j]);
+            for (int j = 0; j < PARTS; ++j)
+                *reinterpret_cast<TO *>(dst + off_o[j]) = from_f32<TO>(o[j]);
         } else {
-            const int left = S - c * kC - 4 * lg - ks * PARTS;
 #pragma unroll
             for (int j = 0; j < PARTS; ++j)
-                if (j < left) dst[j * o_tok] = from_f32<TO>(o[j]);
+                if (j < left) *reinterpret_cast<TO *>(dst + off_o[j]) = from_f32<TO>(o[j]);
         }
     };
 
@@ -456,6 +476,7 @@ __global__ __launch_bounds__(KSPLIT > 1 ? KSPLIT * kWave : kBlock, 2) void delta
 
     offsets(min(kC, S) - 1);
     if constexpr (SHARED) {
+        row_offsets(kC - 1);
         load_rows(0);
         write_rows(0);
         load_rows(1);
