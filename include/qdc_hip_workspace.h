@@ -49,6 +49,25 @@ int32_t qdc_attention_fused(void *out, int32_t out_dtype, const void *q, const v
                             int64_t v_tok, int64_t v_head, int64_t gate_tok, int64_t gate_head,
                             int64_t out_tok, float scale, int32_t dtype, hipStream_t stream);
 
+/* fp32 sums of out = a w^T for an output of few tiles: the inner dimension is cut
+ * into `parts`, and out is [parts][rows][cols], one partial product after the other.
+ * `a` is [rows, inner] bf16, or with a_dtype QDC_BF16X2 in the split form (2 inner
+ * values a row); `w` is [cols, inner] bf16.  ld_a and ld_w in bf16 values.  inner a
+ * multiple of 64 (32 for a split a), cols of 128, strides of 8, parts at most the
+ * steps of 64 values of a, pointers 16-byte aligned (QDC_ERR_SHAPE otherwise). */
+int32_t qdc_linear_parts(float *out, const void *a, const void *w, int64_t rows, int64_t inner,
+                         int64_t cols, int64_t ld_a, int64_t ld_w, int64_t parts, int32_t a_dtype,
+                         hipStream_t stream);
+
+/* residual = x + the sum of `parts` [rows, width] tensors and normed = rms(residual) *
+ * (1 + norm) * mask (mask null: 1): qdc_residual_rmsnorm(_masked) reading the sums of
+ * qdc_linear_parts.  norm is fp32 for out_dtype QDC_F32, else bf16; out_dtype may be
+ * QDC_BF16X2; width 256, 512, 1024 or 2048.  residual may be x; otherwise outputs
+ * overlap neither each other nor an input. */
+int32_t qdc_residual_rms_parts(float *residual, void *normed, const float *x, const float *sums,
+                               int64_t parts, const void *norm, const int32_t *mask, int64_t rows,
+                               int64_t width, float eps, int32_t out_dtype, hipStream_t stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -72,6 +72,9 @@ WORKSPACE_SIGNATURES = {
                           + [_vp, _i64, _vp]),
     "qdc_attention_fused": (_i32, [_vp, _i32, _vp, _vp, _vp, _vp, _vp] + [_i64] * 14
                             + [_f32, _i32, _vp]),
+    "qdc_linear_parts": (_i32, [_vp, _vp, _vp] + [_i64] * 6 + [_i32, _vp]),
+    "qdc_residual_rms_parts": (_i32, [_vp, _vp, _vp, _vp, _i64, _vp, _vp, _i64, _i64, _f32, _i32,
+                                      _vp]),
 }
 
 _lib = None

@@ -20,8 +20,8 @@ residual add (``qdc_residual_rmsnorm``; the last one with the final norm) and,
 before a DeltaNet layer, with its input mask (``qdc_residual_rmsnorm_masked``),
 post-attention residual + RMSNorm, the attention prologue (q/k norm + partial
 RoPE, read straight out of the packed projection), causal attention with its
-masked softmax and output gate in one pass over the heads, the DeltaNet prologue (convolution, SiLU, q/k L2 norm, gates), the gated-delta
-recurrence, the DeltaNet gated RMSNorm reading z inside the packed projection,
+masked softmax and output gate in one pass over the heads, the DeltaNet prologue
+(convolution, SiLU, q/k L2 norm, gates), the gated-delta recurrence, the DeltaNet gated RMSNorm reading z inside the packed projection,
 and SwiGLU reading the packed gate||up GEMM output.  GEMMs run through
 PyTorch-ROCm (hipBLASLt), with fp32 results; attention scores, exponentials and
 their sums are fp32 (the exponentials enter the product with V in the model
@@ -101,6 +101,15 @@ class QwenBackbone:
                 w = torch.cat([w, w.new_zeros((extra, w.shape[1]))], 0)
             return gemm_weight(w, self.mlp_in if mlp else self.gemm_in)
 
+        def residual_stream(key, name, split):
+            """A projection into the residual stream: transposed for the library's
+            product and, in bf16, as the checkpoint has it ([out, in], a copy of our
+            own) for the product cut into parts."""
+            w = dev(weights[name])
+            layer[key] = gemm_weight(w, split)
+            if dtype == torch.bfloat16:
+                layer[key + "_rows"] = w.clone() if w is weights[name] else w
+
         self.embedding = dev(weights["embed_tokens.weight"])
         # the last residual add is fused with the final norm, which writes fp32
         self.final_norm = dev(weights["norm.weight"], torch.float32)
@@ -112,8 +121,8 @@ class QwenBackbone:
                 "input_norm": dev(weights[p + "input_layernorm.weight"]),
                 "post_norm": dev(weights[p + "post_attention_layernorm.weight"]),
                 "gate_up": lin(p + "mlp.gate_proj.weight", p + "mlp.up_proj.weight", mlp=True),
-                "down": lin(p + "mlp.down_proj.weight", mlp=True),
             }
+            residual_stream("down", p + "mlp.down_proj.weight", self.mlp_in)
             if kind == "full_attention":
                 a = p + "self_attn."
                 # q_proj's rows are [q_h; gate_h] per head; regrouped so the packed
@@ -127,8 +136,9 @@ class QwenBackbone:
                                                         dev(weights[a + "v_proj.weight"]),
                                                         qg[:, 1].reshape(H * hd, -1)], 0),
                                              self.gemm_in),
-                             out=lin(a + "o_proj.weight"), q_norm=dev(weights[a + "q_norm.weight"]),
+                             q_norm=dev(weights[a + "q_norm.weight"]),
                              k_norm=dev(weights[a + "k_norm.weight"]))
+                residual_stream("out", a + "o_proj.weight", self.gemm_in)
             elif kind == "linear_attention":
                 a = p + "linear_attn."
                 conv = weights[a + "conv1d.weight"]
@@ -146,8 +156,8 @@ class QwenBackbone:
                     # fixed decay multiplier, computed once in fp32 (src/backbone.jl:160-162)
                     a_decay=(-1.0 * torch.exp(a_log.to(torch.float32))).to(self.device).contiguous(),
                     dt_bias=dev(weights[a + "dt_bias"], torch.float32),
-                    norm=dev(weights[a + "norm.weight"]),
-                    out=lin(a + "out_proj.weight"))
+                    norm=dev(weights[a + "norm.weight"]))
+                residual_stream("out", a + "out_proj.weight", self.gemm_in)
             else:
                 raise ValueError(f"Unsupported layer type {kind}.")
             self.layers.append(layer)
@@ -230,31 +240,54 @@ class QwenBackbone:
             if final_query:
                 mixed = self._final_query_attention(layer, normed, mask32, B, S)
             elif layer["kind"] == "full_attention":
-                mixed = self._full_attention(layer, normed, mask32, B, S)
+                mixed = self._attention_context(layer, normed, mask32, B, S)
             else:
-                mixed = self._delta_attention(layer, normed, B, S)
-            if last and last_only:  # the MLP and the final norm of the last rows only
+                mixed = self._delta_context(layer, normed, B, S)
+            if last and last_only:  # the last rows only from the output projection on
                 h = h.view(B, S, -1)[:, -1].contiguous()
                 if not final_query:
                     mixed = mixed.view(B, S, -1)[:, -1].contiguous()
-            residual, normed = ops.native_residual_rms(h, mixed, layer["post_norm"], cfg.eps,
-                                                       out_dtype=self.mlp_in)
+            if final_query:
+                residual, normed = ops.native_residual_rms(h, mixed, layer["post_norm"], cfg.eps,
+                                                           out_dtype=self.mlp_in)
+            else:
+                residual, normed = self._project_add_norm(h, mixed, layer, "out",
+                                                          layer["post_norm"],
+                                                          out_dtype=self.mlp_in)
             # split inputs: fp32 gate/up for SwiGLU (bf16 there costs ~6x the
             # end-to-end error of the whole split pipeline)
             gate_up = (self._mm32 if self.split else self._mm)(normed, layer["gate_up"])
             inter = gate_up.shape[1] // 2
             act = ops.native_mlp_gate(gate_up[:, :inter], gate_up[:, inter:],
                                       out_dtype=self.mlp_in)
-            down = self._mm32(act, layer["down"])
             nxt = self.final_norm if last else self.layers[i + 1]["input_norm"]
             # residual add of the MLP fused with the next RMSNorm
-            h, normed = ops.native_residual_rms(residual, down, nxt, cfg.eps,
-                                                token_mask=None if last else delta_keep(i + 1),
-                                                out_dtype=None if last else self.gemm_in)
+            h, normed = self._project_add_norm(residual, act, layer, "down", nxt,
+                                               token_mask=None if last else delta_keep(i + 1),
+                                               out_dtype=None if last else self.gemm_in)
         return normed
 
+    def _project_add_norm(self, h, a, layer, name, norm, token_mask=None, out_dtype=None):
+        """A projection into the residual stream, the residual add and the norm that
+        follows: ``(h + a @ W, rms(h + a @ W))``.  Where the projection's output has too
+        few tiles for the chip, its inner dimension is cut into parts that the norm
+        adds up."""
+        rows = layer.get(name + "_rows")
+        if rows is not None:
+            width, inner = rows.shape
+            parts = ops.linear_parts_for(a.shape[0], inner, width, a.shape[1] != inner)
+            if parts:
+                return ops.linear_residual_rms(h, a, rows, norm, self.cfg.eps, parts,
+                                               token_mask=token_mask, out_dtype=out_dtype)
+        return ops.native_residual_rms(h, self._mm32(a, layer[name]), norm, self.cfg.eps,
+                                       token_mask=token_mask, out_dtype=out_dtype)
+
     def _full_attention(self, layer, x, mask32, B, S):
-        """``full_attention`` in the AMDGPU form (``ext/amdgpu_attention.jl:108-178``;
+        return self._mm32(self._attention_context(layer, x, mask32, B, S), layer["out"])
+
+    def _attention_context(self, layer, x, mask32, B, S):
+        """What the output projection of a full-attention layer multiplies:
+        ``full_attention`` in the AMDGPU form (``ext/amdgpu_attention.jl:108-178``;
         generic ``src/backbone.jl:224-262``): q and k normalised and rotated out of
         the packed projection, then scores, masked softmax, the product with v and
         the output gate in one kernel that reads v and the gate inside the
@@ -277,9 +310,8 @@ class QwenBackbone:
         if ops.attention_fused_takes(self.dtype, hd):
             q, k = ops.prepare_heads(q_in, k_in, layer["q_norm"], layer["k_norm"], tables,
                                      cfg.rotary_dim, cfg.eps, seq_len=S)
-            merged = ops.attention_fused(q, k, v_in, gate, mask32, scale, B,
-                                         out_dtype=self.gemm_in or self.dtype)
-            return self._mm32(merged, layer["out"])
+            return ops.attention_fused(q, k, v_in, gate, mask32, scale, B,
+                                       out_dtype=self.gemm_in or self.dtype)
         q, kt, v = ops.attention_prepare(q_in, k_in, v_in, layer["q_norm"], layer["k_norm"],
                                          tables, cfg.rotary_dim, cfg.eps, B)
         scores = self._bmm32(q.view(B * KV, G * S, hd), kt.view(B * KV, hd, S))  # [B*KV, G*S, S]
@@ -287,9 +319,8 @@ class QwenBackbone:
                                       out=scores.view(B, H, S, S) if self.dtype == torch.float32
                                       else None)
         values = self._bmm32(probs.view(B * KV, G * S, S), v.view(B * KV, S, hd))  # [B, H, S, hd]
-        merged = ops.attention_gate(values.view(B, H, S, hd), gate,
-                                    out_dtype=self.gemm_in or self.dtype)
-        return self._mm32(merged, layer["out"])
+        return ops.attention_gate(values.view(B, H, S, hd), gate,
+                                  out_dtype=self.gemm_in or self.dtype)
 
     def _final_query_attention(self, layer, x, mask32, B, S):
         """Final-query attention of the last-token forward: K and V over the
@@ -334,7 +365,11 @@ class QwenBackbone:
         return torch.bmm(a, b, out_dtype=torch.float32)
 
     def _delta_attention(self, layer, x, B, S):
-        """Gated DeltaNet (``src/backbone.jl:284-345``; recurrent form
+        return self._mm32(self._delta_context(layer, x, B, S), layer["out"])
+
+    def _delta_context(self, layer, x, B, S):
+        """What the output projection of a DeltaNet layer multiplies: gated
+        DeltaNet (``src/backbone.jl:284-345``; recurrent form
         ``src/backbone_cpu.jl:680-759``) on an input whose masked tokens the
         producing norm has already zeroed (``native_layer_outputs(...,
         Val(true))``, ``src/backbone.jl:372-376``)."""
@@ -356,7 +391,7 @@ class QwenBackbone:
         z = proj[:, cq:cq + vw].view(T, vh, vd)
         out = ops.native_gated_rms(result.view(T, vh, vd), z, layer["norm"], cfg.eps,
                                    out_dtype=self.gemm_in)
-        return self._mm32(out.view(T, -1), layer["out"])
+        return out.view(T, -1)
 
 
 # ---------------------------------------------------------------- API -------

@@ -344,6 +344,69 @@ def native_residual_rms(x: torch.Tensor, mixed: torch.Tensor, weight: torch.Tens
     return residual, out
 
 
+def linear_parts_for(rows: int, inner: int, width: int, split: bool) -> int:
+    """Into how many parts :func:`linear_residual_rms` cuts the inner dimension of a
+    bf16 product ``[rows, inner] x [inner, width]``, or 0 where one library product
+    is as fast or the kernels do not take the sizes."""
+    slots = 2 * inner if split else inner
+    if width not in (256, 512, 1024, 2048) or slots % 64:
+        return 0
+    # Fewer than 48 steps of 64 leave nothing to cut (2048 to 1024 columns: 16.6 us here,
+    # 15.2 as one product at 300 rows, 22.4 / 24.1 at 1200); below 64 rows the library has
+    # small tiles (33 rows, 3584 to 1024: 13.1 / 11.1), past 120 tiles enough of them
+    # (2400 rows, 152 tiles: 46 / 41; 1800 rows, 120 tiles: 33.5 / 36.4).
+    steps, tiles = slots // 64, -(-rows // 128) * (width // 128)
+    if steps < 48 or rows < 64 or tiles > 120:
+        return 0
+    # Enough workgroups for most of the 256 compute units, and twice as many while the
+    # parts are long (80 tiles of 112 steps: 2 parts 45.3 us, 4 42.9, 8 44.8; of 56 steps:
+    # 30.8, 31.5, 34.8; 40 tiles of 112 steps: 4 parts 28.4, 8 29.7).
+    parts = 1
+    while parts < 8 and (tiles * parts < 160 or
+                         (tiles * parts < 400 and steps >= 56 * parts)):
+        parts *= 2
+    return parts
+
+
+def linear_residual_rms(x: torch.Tensor, a: torch.Tensor, w: torch.Tensor, weight: torch.Tensor,
+                        eps: float, parts: int, token_mask: torch.Tensor | None = None,
+                        out_dtype=None):
+    """``residual = x + a @ w.T``; returns ``(residual, rms(residual))`` as
+    :func:`native_residual_rms` does, for a product of few output tiles: fp32 sums of
+    ``parts`` cuts of the inner dimension, added as the norm reads them.  ``x``
+    float32 ``[rows, width]``, ``w`` bfloat16 ``[width, inner]`` (a checkpoint's
+    layout), ``a`` bfloat16 ``[rows, inner]`` or in the split form ``[rows, 2*inner]``."""
+    _device(x, a, w, weight)
+    if x.dtype != torch.float32 or a.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 \
+            or weight.dtype not in _DTYPES:
+        raise ValueError("x is float32, a and w bfloat16")
+    if x.dim() != 2 or a.dim() != 2 or w.dim() != 2 or not x.is_contiguous() \
+            or a.stride(1) != 1 or w.stride(1) != 1:
+        raise ValueError("x, a and w must be matrices with contiguous rows")
+    rows, width = x.shape
+    inner = w.shape[1]
+    if a.shape[0] != rows or w.shape[0] != width or a.shape[1] not in (inner, 2 * inner):
+        raise ValueError("inconsistent shapes")
+    _vector(weight, width, "weight")
+    split = _is_split(out_dtype)
+    if split and weight.dtype != torch.bfloat16:
+        raise ValueError("the split output takes a bfloat16 weight")
+    keep = _row_mask(token_mask, rows, x)
+    sums = torch.empty((parts, rows, width), dtype=torch.float32, device=x.device)
+    residual = torch.empty_like(x)
+    out = torch.empty((rows, 2 * width if split else width), dtype=weight.dtype, device=x.device)
+    a_code = _lib.QDC_BF16X2 if a.shape[1] == 2 * inner else _lib.QDC_BF16
+    check(lib().qdc_linear_parts(sums.data_ptr(), a.data_ptr(), w.data_ptr(), rows, inner, width,
+                                 a.stride(0) if rows > 1 else a.shape[1], w.stride(0), parts,
+                                 a_code, _stream(x)), "linear_residual_rms")
+    check(lib().qdc_residual_rms_parts(residual.data_ptr(), out.data_ptr(), x.data_ptr(),
+                                       sums.data_ptr(), parts, weight.data_ptr(),
+                                       0 if keep is None else keep.data_ptr(), rows, width, eps,
+                                       _lib.QDC_BF16X2 if split else _DTYPES[weight.dtype],
+                                       _stream(x)), "linear_residual_rms")
+    return residual, out
+
+
 def native_gated_rms(x: torch.Tensor, z: torch.Tensor, weight: torch.Tensor, eps: float,
                      out: torch.Tensor | None = None, out_dtype=None) -> torch.Tensor:
     """``((x*s)*w)*silu(z)`` per ``[tokens, heads, width]`` row, not centred.

@@ -183,3 +183,103 @@ def test_attention_fused_edges(B, S, H, KV, hd, kind, dtype, out):
     bound = spread * (1e-5 if dtype == torch.float32 else 2.0 ** -8 + 1e-5)
     bound = bound + exact.abs() * {"f32": 0.0, "bf16": 2.0 ** -8, "split": 2.0 ** -16}[out] + 1e-30
     assert ((got - exact).abs() <= bound).all(), ((got - exact).abs() / bound).max()
+
+
+def test_linear_parts_validation():
+    lib = _lib.lib()
+
+    def f(out=FAKE, a=BIG, w=BIG, rows=5, inner=128, cols=256, ld_a=128, ld_w=128, parts=2,
+          dt=BF16):
+        return lib.qdc_linear_parts(out, a, w, rows, inner, cols, ld_a, ld_w, parts, dt, None)
+
+    assert f(dt=F32) == -3
+    assert f(inner=96) == -2 and f(cols=192) == -2 and f(ld_a=120) == -2 and f(ld_w=132) == -2
+    assert f(parts=0) == -2 and f(parts=3) == -2 and f(inner=32, ld_a=64, dt=BF16) == -2
+    assert f(dt=X2) == -2                          # a split row holds 2 inner values
+    assert f(a=BIG + 8) == -2 and f(out=FAKE + 4) == -2 and f(rows=1 << 23, ld_a=512) == -2
+    assert f(out=None) == -1 and f(a=None) == -1 and f(w=None) == -1
+    assert f(a=FAKE + 16) == -5 and f(w=FAKE + 16) == -5
+    assert f(rows=0, out=None) == 0
+
+    def g(res=FAKE, normed=FAKE + (1 << 20), x=BIG, sums=BIG, parts=2, norm=BIG, mask=None, rows=5,
+          width=256, odt=BF16):
+        return lib.qdc_residual_rms_parts(res, normed, x, sums, parts, norm, mask, rows, width,
+                                          1e-6, odt, None)
+
+    assert g(odt=7) == -3
+    assert g(width=320) == -2 and g(parts=0) == -2 and g(rows=-1) == -2 and g(x=BIG + 4) == -2
+    for name in ("res", "normed", "x", "sums", "norm"):
+        assert g(**{name: None}) == -1, name
+    for name in ("normed", "sums", "norm", "mask"):
+        assert g(**{name: FAKE + 16}) == -5, name
+    assert g(x=FAKE + 16) == -5 and g(x=FAKE + (1 << 20)) == -5   # x itself is fine for res only
+    assert g(rows=0, res=None) == 0
+
+
+def test_linear_parts_rule():
+    """Parts only where a tile's walk is long and the tiles are few; every choice is one
+    the entry point takes (at least 4 steps of 64 values a part)."""
+    from qdc_amd import ops
+    assert ops.linear_parts_for(63, 3584, 1024, True) == 0
+    assert ops.linear_parts_for(1200, 2048, 1024, False) == 0
+    assert ops.linear_parts_for(16384, 3584, 1024, True) == 0
+    assert ops.linear_parts_for(1200, 3584, 1000, True) == 0
+    assert ops.linear_parts_for(1200, 3584, 1024, True) == 4
+    for rows in (64, 129, 700, 1601):
+        for inner in (32, 64, 96, 480, 2048, 3072, 3584):
+            for split in (False, True):
+                parts = ops.linear_parts_for(rows, inner, 1024, split)
+                slots = inner * (2 if split else 1)
+                assert parts == 0 or (slots % 64 == 0 and (parts == 1 or slots // 64 >= 4 * parts))
+
+
+# rows around a tile of 128 and its wavefronts' 64; parts that do not divide the steps
+LINEAR = [(1, 64, 256, 1), (33, 128, 256, 2), (63, 320, 512, 3), (64, 1024, 1024, 8),
+          (65, 448, 2048, 7), (127, 192, 1024, 2), (128, 64, 512, 1), (129, 576, 256, 4),
+          (300, 704, 1024, 5)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("out", ["f32", "bf16", "split"])
+@pytest.mark.parametrize("split_a", [False, True])
+@pytest.mark.parametrize("rows,inner,width,parts", LINEAR)
+def test_linear_residual_rms_edges(rows, inner, width, parts, split_a, out):
+    """Against 64 bits on the same bf16 values: products are exact in fp32, so the
+    residual stream is within fp32 sums of it (1e-5), the norm within that and its
+    own rounding (bf16 2^-8 per element)."""
+    from qdc_amd import ops
+    g = torch.Generator(device="cuda").manual_seed(rows + inner)
+
+    def randn(*shape):
+        return torch.randn(shape, generator=g, device="cuda")
+
+    x, w = randn(rows, width), (randn(width, inner) * 0.1).bfloat16()
+    a = randn(rows, inner)
+    if split_a:
+        hi = a.bfloat16()
+        lo = (a - hi.float()).bfloat16()
+        a = torch.stack([hi.view(rows, -1, 4), lo.view(rows, -1, 4)], 2).reshape(rows, 2 * inner)
+        exact_a = ops.join_split(a).double()
+    else:
+        a = a.bfloat16()
+        exact_a = a.double()
+    wide = torch.full((rows, a.shape[1] + 8), float("nan"), dtype=torch.bfloat16, device="cuda")
+    wide[:, :a.shape[1]] = a
+    norm = randn(width) * 0.1
+    norm = norm if out == "f32" else norm.bfloat16()
+    mask = (torch.rand(rows, generator=g, device="cuda") > 0.3).int()
+    res, normed = ops.linear_residual_rms(x, wide[:, :a.shape[1]], w, norm, 1e-6, parts,
+                                          token_mask=mask,
+                                          out_dtype=ops.BF16X2 if out == "split" else None)
+    exact = x.double() + exact_a @ w.double().t()
+    assert ((res.double() - exact).abs() <= 1e-5 * exact.abs().max()).all()
+    want = exact * torch.rsqrt(exact.square().mean(-1, keepdim=True) + 1e-6)
+    want = want * (1.0 + norm.double()) * mask[:, None]
+    got = (ops.join_split(normed) if out == "split" else normed).double()
+    rel = 2.0 ** -8 if out == "bf16" else 2.0 ** -16
+    assert ((got - want).abs() <= rel * want.abs() + 2e-5).all()
+    plain = ops.linear_residual_rms(x, a, w, norm, 1e-6, parts,
+                                    out_dtype=ops.BF16X2 if out == "split" else None)
+    assert torch.equal(plain[0], res)
+    assert torch.equal(plain[1][mask.bool()], normed[mask.bool()])
+    assert not normed[~mask.bool()].any()
