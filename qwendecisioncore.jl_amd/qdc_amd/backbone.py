@@ -404,7 +404,7 @@ def check_sequence(model: QwenBackbone, ids, mask) -> None:
     if ids.size == 0:
         raise ValueError("Inputs must not be empty.")
     ops.check_ids(ids, model.vocab)
-    if not np.isin(mask, (0, 1)).all():
+    if not ((mask == 0) | (mask == 1)).all():
         raise ValueError("Mask values must be zero or one.")
 
 
@@ -423,11 +423,16 @@ def _host_sequence(model, ids, mask):
 
 def _device_inputs(model, ids, mask):
     ids, mask = _host_sequence(model, ids, mask)
-    d_ids = torch.from_numpy(ids.astype(np.int32)).to(model.device).view(1, -1)
-    if mask.all():  # nothing masked: the forward skips the masking work
-        return d_ids, None
-    d_mask = torch.from_numpy(mask.astype(np.int32)).to(model.device).view(1, -1)
-    return d_ids, d_mask
+    return _upload(model, ids[None], mask[None])
+
+
+def _upload(model, ids, mask):
+    """Checked host ids and mask ``[B, S]`` to the device as int32, in one copy; the
+    mask only if something is masked (else the forward skips the masking work)."""
+    if mask.all():
+        return torch.from_numpy(ids.astype(np.int32)).to(model.device), None
+    both = torch.from_numpy(np.stack((ids, mask)).astype(np.int32)).to(model.device)
+    return both[0], both[1]
 
 
 def backbone_hidden(model: QwenBackbone, ids, mask, positions=None) -> np.ndarray:
@@ -461,11 +466,8 @@ def native_sequence_start(mask, row: int) -> int:
     rotary attention scores depend only on relative positions."""
     if os.environ.get("QDC_AMDGPU_TRIM_PADDING", "1") != "1":
         return 0
-    row_mask = np.asarray(mask)[row]
-    start = 0
-    while start < row_mask.shape[0] - 1 and row_mask[start] == 0:
-        start += 1
-    return start
+    kept = np.asarray(mask)[row] != 0
+    return int(kept[:-1].argmax()) if kept[:-1].any() else kept.shape[0] - 1
 
 
 def _batch_inputs(model: QwenBackbone, ids, mask, trim: bool = False):
@@ -485,9 +487,7 @@ def _batch_inputs(model: QwenBackbone, ids, mask, trim: bool = False):
             # (ext/metal_batch_forward.jl:113-116, 124-125)
             first = min(native_sequence_start(host_mask, r) for r in range(ids.shape[0]))
             ids, host_mask = ids[:, first:], host_mask[:, first:]
-        d_ids = torch.from_numpy(ids.astype(np.int32)).to(model.device)
-        d_mask = None if host_mask.all() else torch.from_numpy(
-            host_mask.astype(np.int32)).to(model.device)
+        d_ids, d_mask = _upload(model, ids, host_mask)
         return d_ids, d_mask, None
     if ids.dim() != 2 or ids.numel() == 0:
         raise ValueError("Inputs must be a non-empty [batch, sequence] array.")

@@ -87,7 +87,9 @@ def _dtype_code(*tensors) -> int:
 
 
 def _stream(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+    # the raw handle: the Stream object around it took 4.8 us a call, 140 us of the
+    # 950 us a host needs to issue a 4-layer forward
+    return torch._C._cuda_getCurrentRawStream(t.device.index)
 
 
 def _device(*tensors) -> None:
