@@ -68,6 +68,24 @@ int32_t qdc_residual_rms_parts(float *residual, void *normed, const float *x, co
                                int64_t parts, const void *norm, const int32_t *mask, int64_t rows,
                                int64_t width, float eps, int32_t out_dtype, hipStream_t stream);
 
+/* An fp32 projection of few rows with the row work around it: out = in w, or with
+ * swiglu != 0 and w = [gate | up] of 2 cols columns out = silu(in gate) * (in up), where
+ *   input 0: in = a;
+ *   input 1: residual = a + b, in = rms(residual) * (1 + norm) * mask (mask null: 1), as
+ *            qdc_residual_rmsnorm(_masked); residual is [rows, inner];
+ *   input 2: in = the gated norm of every head of head_dim values of a with z = b, as
+ *            qdc_gated_rmsnorm; swiglu must be 0.
+ * inner 128, 256 or 512, cols a multiple of 64, head_dim of 64 that divides inner; rows
+ * ld_a, ld_b, ld_w (of w: [inner, columns]) and ld_out elements apart, multiples of 4;
+ * pointers 16-byte aligned (QDC_ERR_SHAPE otherwise; an input outside 0..2
+ * QDC_ERR_RANGE).  Pointers an input does not use are ignored.  Outputs overlap
+ * neither each other nor an input. */
+int32_t qdc_linear_f32(float *out, float *residual, const float *a, const float *b,
+                       const float *norm, const int32_t *mask, const float *w, int64_t rows,
+                       int64_t inner, int64_t cols, int64_t head_dim, int64_t ld_a, int64_t ld_b,
+                       int64_t ld_w, int64_t ld_out, float eps, int32_t input, int32_t swiglu,
+                       hipStream_t stream);
+
 #ifdef __cplusplus
 }
 #endif

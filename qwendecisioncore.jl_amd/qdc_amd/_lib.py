@@ -75,6 +75,7 @@ WORKSPACE_SIGNATURES = {
     "qdc_linear_parts": (_i32, [_vp, _vp, _vp] + [_i64] * 6 + [_i32, _vp]),
     "qdc_residual_rms_parts": (_i32, [_vp, _vp, _vp, _vp, _i64, _vp, _vp, _i64, _i64, _f32, _i32,
                                       _vp]),
+    "qdc_linear_f32": (_i32, [_vp] * 7 + [_i64] * 8 + [_f32, _i32, _i32, _vp]),
 }
 
 _lib = None

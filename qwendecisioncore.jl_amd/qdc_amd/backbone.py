@@ -161,6 +161,7 @@ class QwenBackbone:
             else:
                 raise ValueError(f"Unsupported layer type {kind}.")
             self.layers.append(layer)
+        self.fused_f32 = self._fused_f32_fits()
 
     @classmethod
     def from_weights(cls, weights: dict, cfg: BackboneConfig, device="cuda:0",
@@ -232,6 +233,8 @@ class QwenBackbone:
                                           self.layers[0]["input_norm"], cfg.eps,
                                           token_mask=delta_keep(0), error_flag=error_flag,
                                           normed_dtype=self.gemm_in)
+        if self.fused_f32 and ops.linear_f32_takes(B * S, self.cfg.hidden, self.cfg.intermediate):
+            return self._forward_small(h, normed, mask32, delta_keep, B, S, last_only)
         for i, layer in enumerate(self.layers):
             last = i + 1 == len(self.layers)
             # the last-token forward's last attention layer attends from the
@@ -267,6 +270,63 @@ class QwenBackbone:
                                                out_dtype=None if last else self.gemm_in)
         return normed
 
+    def _fused_f32_fits(self) -> bool:
+        """Whether every projection of this model has the widths, types and alignments
+        of ``ops.linear_f32``."""
+        cfg = self.cfg
+        if self.dtype != torch.float32 or not self.layers:
+            return False
+        # z is the column block of the packed projection after 2 keys and a value
+        if any("proj" in layer for layer in self.layers) and (
+                cfg.value_dim % 64 or 2 * cfg.key_dim * cfg.key_heads % 4):
+            return False
+        shapes = [(cfg.hidden, cfg.intermediate)] + [
+            tuple(layer[name].shape) for layer in self.layers
+            for name in ("qkv", "proj", "out", "down") if name in layer]
+        read = [self.final_norm] + [
+            layer[name] for layer in self.layers
+            for name in ("input_norm", "post_norm", "norm", "qkv", "proj", "out", "gate_up", "down")
+            if name in layer]
+        return all(ops.linear_f32_takes(1, *shape) for shape in shapes) and \
+            all(t.is_contiguous() and t.data_ptr() % 16 == 0 for t in read)
+
+    def _forward_small(self, h, normed, mask32, delta_keep, B, S, last_only):
+        """:meth:`forward` from the first normalised rows on for a small fp32 model: each
+        norm, the gated norm and SwiGLU run inside the projection they feed or follow
+        (``ops.linear_f32``)."""
+        eps = self.cfg.eps
+        due = None  # the MLP output not yet added to h
+        for i, layer in enumerate(self.layers):
+            last = i + 1 == len(self.layers)
+            attention = layer["kind"] == "full_attention"
+            keep = delta_keep(i)
+            if last and last_only and attention:
+                if due is not None:
+                    h, normed = ops.native_residual_rms(h, due, layer["input_norm"], eps,
+                                                        token_mask=keep)
+                mixed = self._final_query_attention(layer, normed, mask32, B, S)
+                h = h.view(B, S, -1)[:, -1].contiguous()
+            else:
+                w = layer["qkv" if attention else "proj"]
+                if due is None:
+                    proj = ops.linear_f32(normed, w)
+                else:
+                    h, proj = ops.linear_f32(h, w, add=due, weight=layer["input_norm"], eps=eps,
+                                             token_mask=keep)
+                if attention:
+                    x, z = self._attend(layer, proj, mask32, B, S), None
+                else:
+                    x, z = self._recur(layer, proj, B, S)
+                if last and last_only:
+                    x, z, h = (t if t is None else t.view(B, S, -1)[:, -1] for t in (x, z, h))
+                    h = h.contiguous()
+                mixed = ops.linear_f32(x, layer["out"]) if z is None else \
+                    ops.linear_f32(x, layer["out"], z=z, weight=layer["norm"], eps=eps)
+            h, act = ops.linear_f32(h, layer["gate_up"], add=mixed, weight=layer["post_norm"],
+                                    eps=eps, swiglu=True)
+            due = ops.linear_f32(act, layer["down"])
+        return ops.native_residual_rms(h, due, self.final_norm, eps)[1]
+
     def _project_add_norm(self, h, a, layer, name, norm, token_mask=None, out_dtype=None):
         """A projection into the residual stream, the residual add and the norm that
         follows: ``(h + a @ W, rms(h + a @ W))``.  Where the projection's output has too
@@ -296,11 +356,14 @@ class QwenBackbone:
         that with the G = H / KV query heads of a KV head as one ``[G*S, hd]`` block
         both products are plain batched GEMMs, around the softmax and gate
         kernels."""
+        return self._attend(layer, self._mm(x, layer["qkv"]), mask32, B, S)
+
+    def _attend(self, layer, proj, mask32, B, S):
+        """Attention and its output gate from the packed projection ``[T, q|k|v|gate]``."""
         cfg = self.cfg
         hd, H, KV = cfg.head_dim, cfg.heads, cfg.kv_heads
         G = H // KV
         T = B * S
-        proj = self._mm(x, layer["qkv"])                     # [T, q | k | v | gate]
         q_in = proj[:, :H * hd].view(T, H, hd)
         k_in = proj[:, H * hd:(H + KV) * hd].view(T, KV, hd)
         v_in = proj[:, (H + KV) * hd:(H + 2 * KV) * hd].view(T, KV, hd)
@@ -373,12 +436,20 @@ class QwenBackbone:
         ``src/backbone_cpu.jl:680-759``) on an input whose masked tokens the
         producing norm has already zeroed (``native_layer_outputs(...,
         Val(true))``, ``src/backbone.jl:372-376``)."""
+        x, z = self._recur(layer, self._mm(x, layer["proj"]), B, S)
+        vh, vd = self.cfg.value_heads, self.cfg.value_dim
+        out = ops.native_gated_rms(x.view(-1, vh, vd), z.view(-1, vh, vd), layer["norm"],
+                                   self.cfg.eps, out_dtype=self.gemm_in)
+        return out.view(B * S, -1)
+
+    def _recur(self, layer, proj, B, S):
+        """The recurrence's output ``[T, heads*dim]`` and z, inside the packed projection
+        ``[T, qkv | z | a | b (+ zero padding)]``."""
         cfg = self.cfg
         kd, kh, vd, vh = cfg.key_dim, cfg.key_heads, cfg.value_dim, cfg.value_heads
         T = B * S
         kw, vw = kd * kh, vd * vh
         cq = 2 * kw + vw
-        proj = self._mm(x, layer["proj"])  # [T, cq + vw + 2*vh (+ zero padding)]
         # conv + SiLU, q/k L2 norm and the beta/decay gates in one pass; q, k, v
         # are the column blocks of one [T, q|k|v] buffer (one output row per token)
         q, k, v, beta, decay = ops.delta_prologue(proj, layer["conv"], layer["a_decay"],
@@ -388,10 +459,7 @@ class QwenBackbone:
         v, beta, decay = v.view(B, S, vh, vd), beta.view(B, S, vh), decay.view(B, S, vh)
         # recurrence straight into the model dtype the gated norm reads
         result = ops.delta_scan(q, k, v, beta, decay, self.dtype)
-        z = proj[:, cq:cq + vw].view(T, vh, vd)
-        out = ops.native_gated_rms(result.view(T, vh, vd), z, layer["norm"], cfg.eps,
-                                   out_dtype=self.gemm_in)
-        return out.view(T, -1)
+        return result.view(T, vw), proj[:, cq:cq + vw]
 
 
 # ---------------------------------------------------------------- API -------

@@ -283,3 +283,76 @@ def test_linear_residual_rms_edges(rows, inner, width, parts, split_a, out):
     assert torch.equal(plain[0], res)
     assert torch.equal(plain[1][mask.bool()], normed[mask.bool()])
     assert not normed[~mask.bool()].any()
+
+
+def test_linear_f32_validation():
+    lib = _lib.lib()
+    FAR = FAKE + (1 << 30)
+
+    def f(out=FAKE, res=FAR, a=BIG, b=BIG, norm=BIG, mask=None, w=BIG, rows=5, inner=256, cols=128,
+          head=128, ld_a=256, ld_b=256, ld_w=256, ld_out=128, inp=1, swiglu=0):
+        return lib.qdc_linear_f32(out, res, a, b, norm, mask, w, rows, inner, cols, head, ld_a, ld_b,
+                                  ld_w, ld_out, 1e-6, inp, swiglu, None)
+
+    assert f(inp=3) == -4 and f(inp=-1) == -4
+    assert f(inner=192) == -2 and f(cols=96) == -2 and f(ld_a=252) == -2 and f(ld_b=254) == -2
+    assert f(ld_w=124) == -2 and f(ld_out=124) == -2 and f(swiglu=1, ld_w=252) == -2
+    assert f(inp=2, head=96) == -2 and f(inp=2, swiglu=1) == -2 and f(inp=2, head=512) == -2
+    assert f(a=BIG + 4) == -2 and f(res=FAR + 8) == -2 and f(mask=BIG + 1) == -2
+    for name in ("out", "res", "a", "b", "norm", "w"):
+        assert f(**{name: None}) == -1, name
+    for name in ("res", "a", "b", "norm", "mask", "w"):
+        assert f(**{name: FAKE + 16}) == -5, name
+    for name in ("a", "b", "norm", "mask", "w"):
+        assert f(**{name: FAR + 16}) == -5, name
+    assert f(rows=0, out=None) == 0
+
+
+LINEAR_F32 = [(1, 128, 64), (15, 256, 128), (16, 512, 64), (17, 256, 1792), (64, 512, 256),
+              (129, 128, 192), (411, 256, 512)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["rows", "rows_glu", "norm", "norm_masked", "norm_glu", "gated"])
+@pytest.mark.parametrize("rows,inner,cols", LINEAR_F32)
+def test_linear_f32_edges(rows, inner, cols, kind):
+    """Against 64 bits: fp32 sums of at most 512 products and the row operators' own
+    rounding, the repository's fp32 bar of 1e-5 per call and per largest element."""
+    from qdc_amd import ops
+    g = torch.Generator(device="cuda").manual_seed(rows + inner + cols)
+
+    def randn(*shape):
+        return torch.randn(shape, generator=g, device="cuda")
+
+    def strided(t):  # rows inside wider rows
+        wide = torch.full((t.shape[0], t.shape[1] + 12), float("nan"), device="cuda")
+        wide[:, 4:4 + t.shape[1]] = t
+        return wide[:, 4:4 + t.shape[1]]
+
+    glu = kind.endswith("glu")
+    a, b, w = randn(rows, inner), randn(rows, inner), randn(inner, (2 if glu else 1) * cols) * 0.1
+    x, residual = a.double(), None
+    if kind.startswith("norm"):
+        weight, mask = randn(inner) * 0.1, None
+        if kind == "norm_masked":
+            mask = (torch.rand(rows, generator=g, device="cuda") > 0.4).int()
+        residual, got = ops.linear_f32(strided(a), w, add=strided(b), weight=weight, eps=1e-6,
+                                       token_mask=mask, swiglu=glu)
+        assert torch.equal(residual, a + b)
+        x = (a + b).double()
+        x = x * torch.rsqrt(x.square().mean(-1, keepdim=True) + 1e-6) * (1.0 + weight.double())
+        x = x if mask is None else x * mask[:, None]
+    elif kind == "gated":
+        weight = randn(128 if inner > 128 else 64) + 1.0
+        got = ops.linear_f32(strided(a), w, z=strided(b), weight=weight, eps=1e-6)
+        heads = x.view(rows, -1, weight.numel())
+        heads = heads * torch.rsqrt(heads.square().mean(-1, keepdim=True) + 1e-6) * weight.double()
+        x = heads.reshape(rows, inner) * torch.nn.functional.silu(b.double())
+    else:
+        got = ops.linear_f32(strided(a), w, swiglu=glu)
+    want = x @ w.double()
+    if glu:
+        want = torch.nn.functional.silu(want[:, :cols]) * want[:, cols:]
+    err = (got.double() - want)
+    assert err.norm() <= 1e-5 * want.norm()
+    assert err.abs().max() <= 1e-5 * want.abs().max()
