@@ -631,8 +631,8 @@ E2E_BATCH, E2E_SEQ = 8, 2048
 
 def fused_sequence(cfg, dev, tokens, split=None):
     """The fused row-kernel launches of one bf16 forward at `tokens` tokens
-    (gather + first input norm, 2 residual norms per layer, SwiGLU per layer, the
-    attention prologue per full-attention layer, gated norm per DeltaNet layer)
+    (gather + first input norm, 2 residual norms per layer, SwiGLU per layer, q/k
+    norm and RoPE per full-attention layer, gated norm per DeltaNet layer)
     on buffers of the forward's shapes and strides.  `split="mlp"` launches them
     as the forward with split MLP inputs does: the post-attention norm writes
     the split output, SwiGLU reads fp32 gate/up and writes the split output."""
@@ -657,11 +657,8 @@ def fused_sequence(cfg, dev, tokens, split=None):
     hd, nh, kv = cfg.head_dim, cfg.heads, cfg.kv_heads
     qkv = rn((tokens, 2 * hd * nh + 2 * hd * kv), bf)
     qn = rn((hd,), bf)
-    # the layouts the forward writes for the attention products
-    n_seq = tokens // E2E_SEQ
-    prep_out = (torch.empty((n_seq, nh, E2E_SEQ, hd), dtype=bf, device=dev),
-                torch.empty((n_seq, kv, hd, E2E_SEQ), dtype=bf, device=dev),
-                torch.empty((n_seq, kv, E2E_SEQ, hd), dtype=bf, device=dev))
+    q_out = torch.empty((tokens, nh, hd), dtype=bf, device=dev)
+    k_out = torch.empty((tokens, kv, hd), dtype=bf, device=dev)
     tables = ops.rope_tables(E2E_SEQ, cfg.rotary_dim, cfg.rope_theta, dev)
     vw = cfg.value_dim * cfg.value_heads
     cq = 2 * cfg.key_dim * cfg.key_heads + vw
@@ -675,10 +672,10 @@ def fused_sequence(cfg, dev, tokens, split=None):
         ops.native_gather_rms(table, ids, w, 1e-6, hidden=h, normed=normed)
         for kind in cfg.layer_types:
             if kind == "full_attention":
-                ops.attention_prepare(qkv[:, :hd * nh].view(tokens, nh, hd),
-                                      qkv[:, hd * nh:hd * (nh + kv)].view(tokens, kv, hd),
-                                      qkv[:, hd * (nh + kv):hd * (nh + 2 * kv)].view(tokens, kv, hd),
-                                      qn, qn, tables, cfg.rotary_dim, 1e-6, n_seq, out=prep_out)
+                ops.prepare_heads(qkv[:, :hd * nh].view(tokens, nh, hd),
+                                  qkv[:, hd * nh:hd * (nh + kv)].view(tokens, kv, hd), qn, qn,
+                                  tables, cfg.rotary_dim, 1e-6, seq_len=E2E_SEQ, q_out=q_out,
+                                  k_out=k_out)
             else:
                 ops.native_gated_rms(dx, proj[:, cq:cq + vw].view(tokens, cfg.value_heads,
                                                                   cfg.value_dim), wv, 1e-6,
@@ -690,9 +687,9 @@ def fused_sequence(cfg, dev, tokens, split=None):
 
 
 def widened_sequence(cfg, dev, batch, seq):
-    """The widened kernels of one bf16 forward: per full-attention layer the
-    masked softmax and the gate merge, per DeltaNet layer the prologue and the
-    recurrence, on buffers of the forward's shapes."""
+    """The widened kernels of one bf16 forward: per full-attention layer
+    attention with its gate, per DeltaNet layer the prologue and the recurrence,
+    on buffers of the forward's shapes."""
     import torch
     from qdc_amd import ops
     bf, f32 = torch.bfloat16, torch.float32
@@ -701,12 +698,12 @@ def widened_sequence(cfg, dev, batch, seq):
     rn = lambda shape, dt: torch.randn(shape, generator=g, device=dev).to(dt)  # noqa: E731
     T = batch * seq
     H, hd = cfg.heads, cfg.head_dim
-    scores = rn((batch, H, seq, seq), f32)
-    probs = torch.empty(scores.shape, dtype=bf, device=dev)
     mask = None  # as in the forward: no padding
-    values = rn((batch, H, seq, hd), f32)
-    qgate = rn((T, H, 2 * hd), bf)
-    merged = torch.empty((T, H * hd), dtype=bf, device=dev)
+    KV = cfg.kv_heads
+    q_heads, k_heads = rn((T, H, hd), bf), rn((T, KV, hd), bf)
+    packed = rn((T, 2 * (H + KV) * hd), bf)  # [q | k | v | gate]
+    v_heads = packed[:, (H + KV) * hd:(H + 2 * KV) * hd].view(T, KV, hd)
+    gate = packed[:, (H + 2 * KV) * hd:].view(T, H, hd)
     kh, kd, vh, vd = cfg.key_heads, cfg.key_dim, cfg.value_heads, cfg.value_dim
     cq = 2 * kh * kd + vh * vd
     proj = rn((T, cq + vh * vd + 2 * vh), bf)
@@ -722,8 +719,7 @@ def widened_sequence(cfg, dev, batch, seq):
     def run():
         for kind in cfg.layer_types:
             if kind == "full_attention":
-                ops.attention_softmax(scores, mask, scale, out=probs)
-                ops.attention_gate(values, qgate[:, :, hd:], out=merged)
+                ops.attention_fused(q_heads, k_heads, v_heads, gate, mask, scale, batch)
             else:
                 q, k, v, beta, decay = ops.delta_prologue(proj, conv, a_dec, dtb, seq, kh, kd,
                                                           vh, vd, out=outs)
