@@ -465,7 +465,8 @@ __global__ __launch_bounds__(KSPLIT > 1 ? KSPLIT * kWave : kBlock, 2) void delta
             for (int j = 0; j < 4; ++j) part_o[c & 1][ks][j][l] = O[j];
             if (c > 0) store(c - 1, due);
         } else {
-            // over chunk c's tile, whose operands have all left it
+            // over chunk c's tile: every wavefront has read its operands from it before
+            // the last barrier (at the end of step c - 1, or before step 0)
             if (c + 2 < chunks) write_rows(c + 2);
             const float o[4] = {O[0], O[1], O[2], O[3]};
             store(c, o);
@@ -506,6 +507,9 @@ __global__ __launch_bounds__(KSPLIT > 1 ? KSPLIT * kWave : kBlock, 2) void delta
         if (n == 0) fetch_p(x);
         refill();
     }
+    // step 0 writes chunk 2's rows over chunk 0's tile: not before every wavefront
+    // has its operands out of it
+    if constexpr (SHARED) __syncthreads();
     for (int c = 0; c < chunks; ++c) step(c, x);
     if constexpr (!SHARED) {
         __syncthreads();

@@ -107,6 +107,35 @@ def test_delta_scan_ws_edges(B, S, KH, H, kd, vd):
         assert np.abs(got[b] - exp).max() <= 1e-5 * np.abs(exp).max()
 
 
+# whole slices (more than 512) over ten chunks and more with a ragged last one: the LDS
+# tiles and running row pointers of that form are used over and over
+LONG_SCAN = [(5, 187, 16, 16, 128, 128), (5, 193, 8, 16, 64, 128), (9, 171, 16, 16, 32, 64)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,S,KH,H,kd,vd", LONG_SCAN)
+def test_delta_scan_ws_long(B, S, KH, H, kd, vd):
+    """As above; decays spread over 0.001 .. 0.5 a token, so that what a chunk leaves
+    in the state is seen in all that follow."""
+    from oracle import forward
+    from qdc_amd import ops
+    assert B * H * vd // 16 > 512
+    rng = np.random.default_rng(S + kd)
+    q = rng.standard_normal((B, S, KH, kd), dtype=np.float32)
+    k = rng.standard_normal((B, S, KH, kd), dtype=np.float32)
+    q /= np.linalg.norm(q, axis=-1, keepdims=True) * np.float32(np.sqrt(kd))
+    k /= np.linalg.norm(k, axis=-1, keepdims=True)
+    v = rng.standard_normal((B, S, H, vd), dtype=np.float32)
+    beta = rng.random((B, S, H), dtype=np.float32)
+    decay = -np.exp(rng.uniform(np.log(1e-3), np.log(0.5), (B, S, H))).astype(np.float32)
+    got = ops.delta_scan(*(torch.from_numpy(x).cuda() for x in (q, k, v, beta, decay)))
+    got = got.cpu().numpy()
+    for b in range(B):
+        exp = forward.delta_recurrence(q[b], k[b], v[b], beta[b], decay[b])
+        assert normwise(got[b], exp) <= 1e-5
+        assert np.abs(got[b] - exp).max() <= 1e-5 * np.abs(exp).max()
+
+
 def test_attention_fused_validation():
     lib = _lib.lib()
 
