@@ -139,7 +139,11 @@ __global__ __launch_bounds__(kBlock, HD > 128 ? 1 : 2) void attention_fused_bf16
     for (int t = 0; t < TILES; ++t)
 #pragma unroll
         for (int r = 0; r < 16; ++r) o[t][r] = 0.0f;
-    float peak = -FLT_MAX, total = 0.0f;  // this query's running maximum; this lane's sum
+    // What the exponents of this query's scores are taken from, its running maximum
+    // times scale_log2 as rounded: the exponentials and the factors that rescale them
+    // use the same value, which is finite before the first key (where a masked score
+    // is -inf) at every scale.  Then this lane's sum.
+    float base = -FLT_MAX, total = 0.0f;
 
     // operands from LDS: K's piece n of key lq of tile u; V^T's rows 32 t .. 32 t + 31
     // and 16 keys (s of the step), by two transposing reads of 4 keys each per lane
@@ -206,10 +210,10 @@ __global__ __launch_bounds__(kBlock, HD > 128 ? 1 : 2) void attention_fused_bf16
         for (int r = 1; r < 16 * SUBS; ++r) top = fmaxf(top, s[r / 16][r % 16]);
         // a new maximum rescales what is summed so far; one within 2^8 of the old
         // is left, its exponentials are at most 2^8 and lose nothing
-        if (__ballot((top - peak) * a.scale_log2 > 8.0f)) {
-            const float next = fmaxf(peak, swap_max32(top));
-            const float f = __builtin_amdgcn_exp2f((peak - next) * a.scale_log2);
-            peak = next;
+        if (__ballot(__builtin_fmaf(top, a.scale_log2, -base) > 8.0f)) {
+            const float next = fmaxf(base, swap_max32(top) * a.scale_log2);
+            const float f = __builtin_amdgcn_exp2f(base - next);
+            base = next;
             total *= f;
 #pragma unroll
             for (int n = 0; n < TILES; ++n) {
@@ -249,7 +253,6 @@ __global__ __launch_bounds__(kBlock, HD > 128 ? 1 : 2) void attention_fused_bf16
             constexpr int LEAD = 4;  // products between an LDS read and its use
             constexpr int ALL = SUBS * STEPS, PER = 16 / STEPS;
             const bf16_t *k = sk[(t + 1) & 1], *v = sv[t & 1];
-            const float base = peak * a.scale_log2;
             float p[8];
             bf16x8 kf[ALL], vf[ALL], pf[2 * SUBS];
             f32x16 next[SUBS] = {};  // past the last step: of old rows, not used

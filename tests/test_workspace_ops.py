@@ -214,6 +214,53 @@ def test_attention_fused_edges(B, S, H, KV, hd, kind, dtype, out):
     assert ((got - exact).abs() <= bound).all(), ((got - exact).abs() / bound).max()
 
 
+def attention_exact(q, k, v, gate, mask, scale, B):
+    """What ``ops.attention_fused`` gives, in 64 bits on the same inputs, and the gated
+    weighted mean of |v|, ``[B, S, H, hd]``; also the scaled scores ``[B, H, S, S]`` with
+    -inf at the keys a query does not see."""
+    H, KV = q.shape[1], k.shape[1]
+    q, k, v, gate = (x.cpu().double().view(B, -1, x.shape[1], x.shape[2]).transpose(1, 2)
+                     for x in (q, k, v, gate))
+    k, v = (x.repeat_interleave(H // KV, 1) for x in (k, v))
+    S = q.shape[2]
+    see = torch.ones(S, S, dtype=torch.bool).tril()[None, None]
+    if mask is not None:
+        see = see & mask.cpu().bool()[:, None, None, :]
+    scores = q @ k.transpose(2, 3) * scale
+    low = -torch.finfo(torch.float32).max
+    p = torch.softmax(scores.masked_fill(~see, low), -1)
+    out = [(torch.sigmoid(gate) * (p @ x)).transpose(1, 2) for x in (v, v.abs())]
+    return out[0], out[1], scores.masked_fill(~see, -torch.inf)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("scale", [0.6, 0.75, 1.0, 8.0])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("B,S,H,KV,hd,kind", [(2, 200, 4, 2, 64, "prefix"), (1, 161, 4, 1, 256, "none"),
+                                              (1, 200, 3, 1, 128, "first")])
+def test_attention_fused_scales(B, S, H, KV, hd, kind, dtype, scale):
+    """Queries scaled beforehand, up to scale 1 and beyond; masked prefixes longer than a
+    step of 64 keys, after which queries see their first key, and queries that see
+    none.  Bounds as in the test of the edges (fp32 output)."""
+    from qdc_amd import ops
+    rng = np.random.default_rng(S + H)
+    T = B * S
+    q, k, v, gate = (torch.from_numpy(rng.standard_normal((T, n, hd), dtype=np.float32))
+                     for n in (H, KV, KV, H))
+    q, k, v, gate = (x.to(dtype).cuda() for x in (q * (2.0 * hd ** -0.5 / scale), k, v, gate))
+    mask = None
+    if kind != "none":
+        m = np.ones((B, S), np.int32)
+        m[:, :(100 if kind == "prefix" else S - 1)] = 0
+        mask = torch.from_numpy(m).cuda()
+    got = ops.attention_fused(q, k, v, gate, mask, scale, B, out_dtype=torch.float32)
+    got = got.double().cpu().view(B, S, H, hd)
+    exact, spread, _ = attention_exact(q, k, v, gate, mask, scale, B)
+    bound = spread * (1e-5 if dtype == torch.float32 else 2.0 ** -8 + 1e-5) + 1e-30
+    assert torch.isfinite(got).all()
+    assert ((got - exact).abs() <= bound).all(), ((got - exact).abs() / bound).max()
+
+
 def test_linear_parts_validation():
     lib = _lib.lib()
 
