@@ -41,7 +41,9 @@ int32_t qdc_delta_scan_ws(void *out, int32_t out_dtype, const float *q, const fl
  * are views of rows of head_dim contiguous elements with their strides between
  * tokens and heads in elements; out_dtype may also be QDC_BF16X2.  head_dim 64,
  * 128 or 256; all strides multiples of 16 bytes and all pointers 16-byte aligned
- * (QDC_ERR_SHAPE otherwise).  out may not overlap any input. */
+ * (QDC_ERR_SHAPE otherwise).  scale is positive, and scale * log2(e) finite
+ * (QDC_ERR_RANGE otherwise; qdc_attention_softmax takes any scale).  out may not
+ * overlap any input. */
 int32_t qdc_attention_fused(void *out, int32_t out_dtype, const void *q, const void *k,
                             const void *v, const void *gate, const int32_t *mask, int64_t batch,
                             int64_t seq, int64_t heads, int64_t kv_heads, int64_t head_dim,

@@ -569,6 +569,9 @@ extern "C" int32_t qdc_attention_fused(void *out, int32_t out_dtype, const void 
                                        hipStream_t stream) {
     const bool split = out_dtype == QDC_BF16X2;
     if (!(valid_dtype(out_dtype) || split) || !valid_dtype(dtype)) return QDC_ERR_DTYPE;
+    // a row's maximum is that of its unscaled scores
+    const float scale_log2 = scale * 1.4426950408889634f;
+    if (!(scale_log2 > 0.0f && scale_log2 < __builtin_inff())) return QDC_ERR_RANGE;
     if (batch < 0 || seq < 0 || heads <= 0 || kv_heads <= 0 || heads % kv_heads)
         return QDC_ERR_SHAPE;
     if (head_dim != 64 && head_dim != 128 && head_dim != 256) return QDC_ERR_SHAPE;
@@ -622,7 +625,7 @@ extern "C" int32_t qdc_attention_fused(void *out, int32_t out_dtype, const void 
     const int64_t blocks = dtype == QDC_BF16 ? ceil_div(units, (int64_t)4) : units;
     if (blocks > 65535) return QDC_ERR_SHAPE;
     a.units = (int)units;
-    a.scale_log2 = scale * 1.4426950408889634f;
+    a.scale_log2 = scale_log2;
     const dim3 grid((uint32_t)(batch * kv_heads), (uint32_t)blocks);
 #define QDC_ATTENTION(HD, TO)                                                                   \
     if (dtype == QDC_BF16)                                                                      \

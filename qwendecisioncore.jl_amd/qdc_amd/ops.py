@@ -879,11 +879,11 @@ def attention_fused(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, gate: tor
                     out_dtype=None) -> torch.Tensor:
     """Causal attention and its output gate in one pass over prepared heads: what
     :func:`attention_softmax` and :func:`attention_gate` give around two batched
-    products, without the score matrix.  ``q`` and ``gate`` ``[T, H, hd]``, ``k``
-    and ``v`` ``[T, KV, hd]`` (views with contiguous rows) of ``batch`` sequences of
-    ``T // batch`` tokens, ``mask`` int32 ``[batch, T // batch]`` or None ->
-    ``[T, H*hd]`` in ``out_dtype`` (default: q's dtype; ``BF16X2`` writes
-    ``[T, 2*H*hd]``)."""
+    products, without the score matrix, for a positive ``scale``.  ``q`` and ``gate``
+    ``[T, H, hd]``, ``k`` and ``v`` ``[T, KV, hd]`` (views with contiguous rows) of
+    ``batch`` sequences of ``T // batch`` tokens, ``mask`` int32
+    ``[batch, T // batch]`` or None -> ``[T, H*hd]`` in ``out_dtype`` (default: q's
+    dtype; ``BF16X2`` writes ``[T, 2*H*hd]``)."""
     _device(q, k, v, gate)
     code = _dtype_code(q, k, v, gate)
     if q.dim() != 3 or k.dim() != 3 or gate.shape != q.shape or v.shape != k.shape:

@@ -214,6 +214,16 @@ def test_attention_fused_edges(B, S, H, KV, hd, kind, dtype, out):
     assert ((got - exact).abs() <= bound).all(), ((got - exact).abs() / bound).max()
 
 
+def test_attention_fused_scale_validation():
+    """The running maximum is taken before the scale: a scale that is not positive and
+    finite (with its log2(e) factor) is refused before anything else is looked at."""
+    lib = _lib.lib()
+    for scale in (0.0, -0.125, float("nan"), float("inf"), -float("inf"), 3e38):
+        status = lib.qdc_attention_fused(None, BF16, BIG, BIG, BIG, BIG, None, 2, 33, 4, 2, 64, 256,
+                                         64, 128, 64, 128, 64, 256, 64, 256, scale, BF16, None)
+        assert status == -4, scale
+
+
 def attention_exact(q, k, v, gate, mask, scale, B):
     """What ``ops.attention_fused`` gives, in 64 bits on the same inputs, and the gated
     weighted mean of |v|, ``[B, S, H, hd]``; also the scaled scores ``[B, H, S, S]`` with
