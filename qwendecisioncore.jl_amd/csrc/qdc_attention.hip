@@ -271,11 +271,6 @@ struct Gate {
     FastDiv seq;
 };
 
-__device__ __forceinline__ float sigmoid_ref(float x) {
-    // native_sigmoid(x) = 1/(1 + exp(-x)) (src/backbone.jl:196)
-    return 1.0f / (1.0f + expf(-x));
-}
-
 // One thread per 8 elements of one (token, head) row: 4 in each half of the row.
 template <typename TG, typename TO>
 __global__ __launch_bounds__(kBlock) void gate_merge_fast(Gate a) {
@@ -303,8 +298,8 @@ __global__ __launch_bounds__(kBlock) void gate_merge_fast(Gate a) {
     unpack(gf1, g1);
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-        v0[j] = v0[j] * sigmoid_ref(g0[j]);
-        v1[j] = v1[j] * sigmoid_ref(g1[j]);
+        v0[j] = v0[j] * sigmoid(g0[j]);
+        v1[j] = v1[j] * sigmoid(g1[j]);
     }
     store_frag<4>(op, v0);
     store_frag<4>(op + half, v1);
@@ -325,7 +320,7 @@ __global__ __launch_bounds__(kBlock) void gate_merge_general(Gate a) {
     const float gv = to_f32(reinterpret_cast<const TG *>(
         a.gate)[(int64_t)t * a.gate_tok + (int64_t)h * a.gate_head + r]);
     put_elem(reinterpret_cast<TO *>(a.out), (int64_t)t * a.out_tok + (int64_t)h * dim + r,
-             v * sigmoid_ref(gv));
+             v * sigmoid(gv));
 }
 
 }  // namespace

@@ -51,27 +51,6 @@ struct Attention {
     float scale_log2;     // scale * log2(e)
 };
 
-// sigmoid(x) to fp32 rounding: exp(-x) = 2^t (1 + r ln 2) with t + r = -x log2(e)
-// carried in two terms, and one Newton step on the hardware reciprocal.
-__device__ __forceinline__ float sigmoid_f32(float x) {
-    const float n = fmaxf(fminf(-x, 88.0f), -100.0f);
-    const float t = n * 1.44269504f;
-    const float r = __builtin_fmaf(n, 1.44269504f, -t) + n * 1.92596299e-8f;
-    const float e2 = __builtin_amdgcn_exp2f(t);
-    const float d = 1.0f + __builtin_fmaf(e2, r * 0.693147181f, e2);
-    const float q = __builtin_amdgcn_rcpf(d);
-    const float y = __builtin_fmaf(__builtin_fmaf(-d, q, 1.0f), q, q);
-    return x == x ? y : x;
-}
-
-// The gate factor of an output of type TO: for bf16 outputs, of one term or two,
-// exp2 of the rounded product is far below their rounding (relative error
-// |x| 2^-24 against 2^-9 and 2^-17).
-template <typename TO> __device__ __forceinline__ float sigmoid_gate(float x) {
-    return __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(x * -1.4426950408889634f));
-}
-template <> __device__ __forceinline__ float sigmoid_gate<float>(float x) { return sigmoid_f32(x); }
-
 __device__ __forceinline__ float swap_max32(float v) {
     const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
     return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
@@ -339,8 +318,8 @@ __global__ __launch_bounds__(kBlock, HD > 128 ? 1 : 2) void attention_fused_bf16
                 const auto r = __builtin_amdgcn_permlane32_swap(
                     __float_as_uint(o[t][8 * i + j]), __float_as_uint(o[t][8 * i + 4 + j]), false,
                     false);
-                y[j] = __uint_as_float(r[0]) * inv * sigmoid_gate<TO>(g[j]);
-                y[4 + j] = __uint_as_float(r[1]) * inv * sigmoid_gate<TO>(g[4 + j]);
+                y[j] = __uint_as_float(r[0]) * inv * sigmoid(g[j]);
+                y[4 + j] = __uint_as_float(r[1]) * inv * sigmoid(g[4 + j]);
             }
             store_frag<8>(op + 32 * t + 16 * i, y);
         }
@@ -545,7 +524,7 @@ __global__ __launch_bounds__(kBlock, 1) void attention_fused_f32(Attention a) {
                     float v = part[0][wv][4 * i + j][l];
 #pragma unroll
                     for (int w = 1; w < NW; ++w) v += part[w][wv][4 * i + j][l];
-                    y[j] = v * sigmoid_gate<TO>(g[j]);
+                    y[j] = v * sigmoid(g[j]);
                 }
                 store_frag<4>(op + 32 * (t0 + wv) + 8 * i, y);
             }

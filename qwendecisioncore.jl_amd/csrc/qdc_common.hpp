@@ -314,6 +314,9 @@ __device__ __forceinline__ float silu(float x) {
     return x * __builtin_amdgcn_rcpf(1.0f + e);
 }
 
+// native_sigmoid(x) = 1/(1 + exp(-x)) (src/backbone.jl:196), of the attention gate.
+__device__ __forceinline__ float sigmoid(float x) { return 1.0f / (1.0f + expf(-x)); }
+
 // ------------------------------------------------------ integer division --
 // Division of n < 2^31 by a fixed divisor d >= 1 with one multiply-high, add
 // and shift (Granlund & Montgomery, "Division by invariant integers using

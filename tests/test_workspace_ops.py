@@ -271,6 +271,28 @@ def test_attention_fused_scales(B, S, H, KV, hd, kind, dtype, scale):
     assert ((got - exact).abs() <= bound).all(), ((got - exact).abs() / bound).max()
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("out", ["f32", "bf16", "split"])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("hd", [64, 128, 256])
+def test_attention_fused_gate(hd, dtype, out):
+    """Sequences of one token and queries of zeros weigh their key by exactly 1: what is
+    left is the output gate, and that is the gate merge's, bit for bit, over the whole
+    range."""
+    from qdc_amd import ops
+    T, H = 300, 2
+    g = torch.Generator(device="cuda").manual_seed(hd)
+    v = torch.randn((T, H, hd), generator=g, device="cuda").to(dtype)
+    gate = torch.empty((T, H, hd), device="cuda").uniform_(-100, 100, generator=g)
+    gate[1::2] *= 0.1
+    gate[0, 0, :6] = torch.tensor([float("inf"), -float("inf"), float("nan"), 0.0, 89.0, -89.0])
+    gate = gate.to(dtype)
+    odt = {"f32": torch.float32, "bf16": torch.bfloat16, "split": ops.BF16X2}[out]
+    got = ops.attention_fused(torch.zeros_like(v), v, v, gate, None, hd ** -0.5, T, out_dtype=odt)
+    want = ops.attention_gate(v.float().view(T, H, 1, hd), gate, out_dtype=odt).view_as(got)
+    assert torch.equal(torch.nan_to_num(got, nan=1e30), torch.nan_to_num(want, nan=1e30))
+
+
 def test_linear_parts_validation():
     lib = _lib.lib()
 
