@@ -103,12 +103,15 @@ class QwenBackbone:
 
         def residual_stream(key, name, split):
             """A projection into the residual stream: transposed for the library's
-            product and, in bf16, as the checkpoint has it ([out, in], a copy of our
-            own) for the product cut into parts."""
-            w = dev(weights[name])
+            product and, where some row count takes the product cut into parts, as the
+            checkpoint has it ([out, in], a copy of our own)."""
+            src = weights[name]
+            w = dev(src)
             layer[key] = gemm_weight(w, split)
-            if dtype == torch.bfloat16:
-                layer[key + "_rows"] = w.clone() if w is weights[name] else w
+            if dtype == torch.bfloat16 and ops.linear_parts_fits(w.shape[1], w.shape[0],
+                                                                 bool(split)):
+                shared = isinstance(src, torch.Tensor) and w.data_ptr() == src.data_ptr()
+                layer[key + "_rows"] = w.clone() if shared else w
 
         self.embedding = dev(weights["embed_tokens.weight"])
         # the last residual add is fused with the final norm, which writes fp32

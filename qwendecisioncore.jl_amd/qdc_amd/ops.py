@@ -346,19 +346,26 @@ def native_residual_rms(x: torch.Tensor, mixed: torch.Tensor, weight: torch.Tens
     return residual, out
 
 
+def linear_parts_fits(inner: int, width: int, split: bool) -> bool:
+    """Whether :func:`linear_parts_for` cuts a product of these sizes at any row count."""
+    slots = 2 * inner if split else inner
+    # Fewer than 48 steps of 64 leave nothing to cut (2048 to 1024 columns: 16.6 us here,
+    # 15.2 as one product at 300 rows, 22.4 / 24.1 at 1200).
+    return width in (256, 512, 1024, 2048) and slots % 64 == 0 and slots // 64 >= 48
+
+
 def linear_parts_for(rows: int, inner: int, width: int, split: bool) -> int:
     """Into how many parts :func:`linear_residual_rms` cuts the inner dimension of a
     bf16 product ``[rows, inner] x [inner, width]``, or 0 where one library product
     is as fast or the kernels do not take the sizes."""
-    slots = 2 * inner if split else inner
-    if width not in (256, 512, 1024, 2048) or slots % 64:
+    if not linear_parts_fits(inner, width, split):
         return 0
-    # Fewer than 48 steps of 64 leave nothing to cut (2048 to 1024 columns: 16.6 us here,
-    # 15.2 as one product at 300 rows, 22.4 / 24.1 at 1200); below 64 rows the library has
-    # small tiles (33 rows, 3584 to 1024: 13.1 / 11.1), past 120 tiles enough of them
-    # (2400 rows, 152 tiles: 46 / 41; 1800 rows, 120 tiles: 33.5 / 36.4).
+    # Below 64 rows the library has small tiles (33 rows, 3584 to 1024: 13.1 / 11.1), past
+    # 120 tiles enough of them (2400 rows, 152 tiles: 46 / 41; 1800 rows, 120 tiles: 33.5 /
+    # 36.4).
+    slots = 2 * inner if split else inner
     steps, tiles = slots // 64, -(-rows // 128) * (width // 128)
-    if steps < 48 or rows < 64 or tiles > 120:
+    if rows < 64 or tiles > 120:
         return 0
     # Enough workgroups for most of the 256 compute units, and twice as many while the
     # parts are long (80 tiles of 112 steps: 2 parts 45.3 us, 4 42.9, 8 44.8; of 56 steps:

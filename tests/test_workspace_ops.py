@@ -341,6 +341,32 @@ def test_linear_parts_rule():
                 assert parts == 0 or (slots % 64 == 0 and (parts == 1 or slots // 64 >= 4 * parts))
 
 
+@pytest.mark.parametrize("split", [False, "mlp", "all"])
+@pytest.mark.parametrize("hidden,inner,vw", [(1024, 3584, 2048), (1024, 3072, 3072), (768, 3584, 2048),
+                                             (256, 768, 1536)])
+def test_rows_kept_where_the_rule_cuts(hidden, inner, vw, split):
+    """A model holds a projection into the residual stream in the checkpoint's layout,
+    beside the transposed one, only where some row count reads it, and as its own
+    copy."""
+    from qdc_amd import backbone, config, ops, weights
+    cfg = config.BackboneConfig(hidden=hidden, head_dim=64, heads=vw // 64, kv_heads=1, key_heads=1,
+                                value_heads=vw // 64, key_dim=64, value_dim=64, eps=1e-6,
+                                rope_theta=1e7, rotary_dim=16, intermediate=inner, vocab=8,
+                                layer_types=("linear_attention", "full_attention"))
+    w = {n: torch.zeros(s, dtype=torch.bfloat16) for n, s in weights.all_shapes(cfg).items()}
+    model = backbone.QwenBackbone.from_weights(w, cfg, "cpu", torch.bfloat16, split_gemm_inputs=split)
+    for i, layer in enumerate(model.layers):
+        for key, name, width, two in (
+                ("down", "mlp.down_proj", inner, bool(split)),
+                ("out", ("linear_attn.out_proj", "self_attn.o_proj")[i], vw, split == "all")):
+            ever = any(ops.linear_parts_for(rows, width, hidden, two) for rows in range(1, 4000))
+            assert (key + "_rows" in layer) == ever
+            if ever:
+                rows = layer[key + "_rows"]
+                src = w[f"layers.{i}.{name}.weight"]
+                assert rows.shape == (hidden, width) and rows.data_ptr() != src.data_ptr()
+
+
 # rows around a tile of 128 and its wavefronts' 64; parts that do not divide the steps
 LINEAR = [(1, 64, 256, 1), (33, 128, 256, 2), (63, 320, 512, 3), (64, 1024, 1024, 8),
           (65, 448, 2048, 7), (127, 192, 1024, 2), (128, 64, 512, 1), (129, 576, 256, 4),
