@@ -336,7 +336,9 @@ class QwenBackbone:
         few tiles for the chip, its inner dimension is cut into parts that the norm
         adds up."""
         rows = layer.get(name + "_rows")
-        if rows is not None:
+        # a norm weight is the caller's own tensor where nothing had to be converted, at
+        # any address; the other operands are allocations of ours
+        if rows is not None and norm.data_ptr() % 16 == 0:
             width, inner = rows.shape
             parts = ops.linear_parts_for(a.shape[0], inner, width, a.shape[1] != inner)
             if parts:

@@ -419,6 +419,35 @@ def test_linear_residual_rms_edges(rows, inner, width, parts, split_a, out):
     assert not normed[~mask.bool()].any()
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_forward_takes_unaligned_weights(dtype):
+    """Weights that are views into one buffer, not on 16 bytes, as a checkpoint reader
+    may hand them over: a forward at a size of the cut product (bf16) and of the small
+    fp32 products gives what aligned weights give, up to the order of sums (one bf16
+    rounding, 2^-8, may go the other way)."""
+    from qdc_amd import backbone, config, ops, weights
+    inner = 3072 if dtype == torch.bfloat16 else 512
+    cfg = config.BackboneConfig(hidden=256, head_dim=64, heads=4, kv_heads=1, key_heads=2, value_heads=2,
+                                key_dim=64, value_dim=64, eps=1e-6, rope_theta=1e7, rotary_dim=16,
+                                intermediate=inner, vocab=64,
+                                layer_types=("linear_attention", "full_attention"))
+    if dtype == torch.bfloat16:
+        assert ops.linear_parts_for(70, inner, 256, False)
+    aligned = weights.random_device_weights(cfg, seed=5, dtype=dtype, std=0.05)
+    flat = torch.empty(sum(t.numel() + 8 for t in aligned.values()) + 8, dtype=dtype, device="cuda")
+    shifted, at = {}, 1
+    for name, t in aligned.items():
+        shifted[name] = flat[at:at + t.numel()].view(t.shape).copy_(t)
+        at += (t.numel() + 7) // 8 * 8
+    assert all(t.data_ptr() % 16 for t in shifted.values())
+    ids = torch.arange(70, dtype=torch.int32, device="cuda").remainder(64).view(1, 70)
+    states = [backbone.batch_backbone_states(backbone.QwenBackbone.from_weights(w, cfg, "cuda", dtype),
+                                             ids, None) for w in (aligned, shifted)]
+    bar = 1e-5 if dtype == torch.float32 else 2.0 ** -8
+    assert normwise(states[1].cpu().numpy(), states[0].cpu().numpy()) <= bar
+
+
 def test_linear_f32_validation():
     lib = _lib.lib()
     FAR = FAKE + (1 << 30)
