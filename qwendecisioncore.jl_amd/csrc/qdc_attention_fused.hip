@@ -558,6 +558,9 @@ extern "C" int32_t qdc_attention_fused(void *out, int32_t out_dtype, const void 
     const int64_t tokens = batch * seq, lim = (int64_t)1 << 31;
     if (batch >= lim || seq >= lim / 64 || heads >= lim / 64 || batch * kv_heads >= lim / kBlock)
         return QDC_ERR_SHAPE;
+    const int64_t units = heads / kv_heads * ceil_div(seq, (int64_t)kQ);
+    const int64_t blocks = dtype == QDC_BF16 ? ceil_div(units, (int64_t)4) : units;
+    if (blocks > 65535) return QDC_ERR_SHAPE;
     // 16-byte pieces of every input, groups of 4 of the output
     const int64_t strides16[] = {q_tok, q_head, k_tok, k_head, v_tok, v_head};
     const int64_t es = elem_size(dtype);
@@ -600,9 +603,6 @@ extern "C" int32_t qdc_attention_fused(void *out, int32_t out_dtype, const void 
     a.H = (int)heads;
     a.KV = (int)kv_heads;
     a.G = (int)(heads / kv_heads);
-    const int64_t units = a.G * ceil_div(seq, (int64_t)kQ);
-    const int64_t blocks = dtype == QDC_BF16 ? ceil_div(units, (int64_t)4) : units;
-    if (blocks > 65535) return QDC_ERR_SHAPE;
     a.units = (int)units;
     a.scale_log2 = scale_log2;
     const dim3 grid((uint32_t)(batch * kv_heads), (uint32_t)blocks);

@@ -375,7 +375,7 @@ class QwenBackbone:
         gate = proj[:, (H + 2 * KV) * hd:].view(T, H, hd)
         tables = self.rope_tables(S) if cfg.rotary_dim else None
         scale = float(np.float32(1) / np.sqrt(np.float32(hd)))      # inv(sqrt(Float32(dim)))
-        if ops.attention_fused_takes(self.dtype, hd):
+        if ops.attention_fused_takes(self.dtype, hd, B, S, H, KV):
             q, k = ops.prepare_heads(q_in, k_in, layer["q_norm"], layer["k_norm"], tables,
                                      cfg.rotary_dim, cfg.eps, seq_len=S)
             return ops.attention_fused(q, k, v_in, gate, mask32, scale, B,

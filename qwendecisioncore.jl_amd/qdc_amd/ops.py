@@ -876,9 +876,16 @@ def attention_gate(values: torch.Tensor, gate: torch.Tensor, out_dtype=None,
     return out
 
 
-def attention_fused_takes(dtype: torch.dtype, head_dim: int) -> bool:
-    """Whether :func:`attention_fused` has a kernel for these heads."""
-    return dtype in _DTYPES and head_dim in (64, 128, 256)
+def attention_fused_takes(dtype: torch.dtype, head_dim: int, batch: int, seq: int, heads: int,
+                          kv_heads: int) -> bool:
+    """Whether :func:`attention_fused` has a kernel for these heads and its grid, a
+    workgroup per KV head of a sequence and 4 (fp32: 1) blocks of 32 queries of a head,
+    holds them."""
+    if dtype not in _DTYPES or head_dim not in (64, 128, 256):
+        return False
+    units = heads // kv_heads * -(-seq // 32)
+    return batch * kv_heads < 1 << 23 and \
+        (-(-units // 4) if dtype == torch.bfloat16 else units) < 1 << 16
 
 
 def attention_fused(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, gate: torch.Tensor,

@@ -224,6 +224,28 @@ def test_attention_fused_scale_validation():
         assert status == -4, scale
 
 
+def test_attention_fused_limits():
+    """The forward takes the kernel exactly where its grid fits: beyond, the form with a
+    score matrix, which took these sizes before."""
+    from qdc_amd import ops
+    lib = _lib.lib()
+    # (batch, seq, heads, kv_heads); a group of 128 heads over one KV head of 16384 tokens
+    # is 65536 units of 32 queries, one more than the grid holds in fp32
+    sizes = [(1, 16384, 128, 1), (1, 16352, 128, 1), (1, 65535, 128, 1), (1, 65536, 128, 1),
+             (1 << 22, 2, 2, 2), ((1 << 22) - 1, 2, 2, 2), (8, 2048, 8, 2), (1, 1 << 25, 8, 2)]
+    for dtype, code in ((torch.float32, F32), (torch.bfloat16, BF16)):
+        for hd in (64, 96, 128, 256):
+            for B, S, H, KV in sizes:
+                status = lib.qdc_attention_fused(None, code, BIG, BIG, BIG, BIG, None, B, S, H, KV, hd,
+                                                 H * hd, hd, KV * hd, hd, KV * hd, hd, H * hd, hd,
+                                                 H * hd, 0.125, code, None)
+                assert status in (-1, -2)   # -1: sizes taken, the null pointer refused
+                assert ops.attention_fused_takes(dtype, hd, B, S, H, KV) == (status == -1), (hd, B, S)
+    assert not ops.attention_fused_takes(torch.float32, 64, *sizes[0])
+    assert ops.attention_fused_takes(torch.bfloat16, 64, *sizes[0])
+    assert not ops.attention_fused_takes(torch.float16, 64, 1, 1, 1, 1)
+
+
 def attention_exact(q, k, v, gate, mask, scale, B):
     """What ``ops.attention_fused`` gives, in 64 bits on the same inputs, and the gated
     weighted mean of |v|, ``[B, S, H, hd]``; also the scaled scores ``[B, H, S, S]`` with
