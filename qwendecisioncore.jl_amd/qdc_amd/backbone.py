@@ -540,7 +540,7 @@ def native_sequence_start(mask, row: int) -> int:
     if os.environ.get("QDC_AMDGPU_TRIM_PADDING", "1") != "1":
         return 0
     kept = np.asarray(mask)[row] != 0
-    return int(kept[:-1].argmax()) if kept[:-1].any() else kept.shape[0] - 1
+    return int(kept[:-1].argmax()) if kept[:-1].any() else max(kept.shape[0] - 1, 0)
 
 
 def _batch_inputs(model: QwenBackbone, ids, mask, trim: bool = False):

@@ -301,3 +301,17 @@ def test_parameter_vectors_checked_before_launch(no_launch):
     for i, call in enumerate(bad):
         with pytest.raises(ValueError):
             call()
+
+
+def test_sequence_start_counts_leading_masked_tokens():
+    """``native_sequence_start`` against the token-by-token count it stands for: leading
+    zeros, never past the last token; rows of no token or one start at 0."""
+    from qdc_amd.backbone import native_sequence_start
+    rng = np.random.default_rng(3)
+    for n in range(9):
+        masks = [np.zeros(n, int), np.ones(n, int)] + [rng.integers(0, 2, n) for _ in range(40)]
+        for r, row in enumerate(masks):
+            start = 0
+            while start < n - 1 and row[start] == 0:
+                start += 1
+            assert native_sequence_start(np.stack(masks), r) == start, (n, row)
