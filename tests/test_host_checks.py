@@ -306,6 +306,7 @@ def test_parameter_vectors_checked_before_launch(no_launch):
 def test_sequence_start_counts_leading_masked_tokens():
     """``native_sequence_start`` against the token-by-token count it stands for: leading
     zeros, never past the last token; rows of no token or one start at 0."""
+    import numpy as np
     from qdc_amd.backbone import native_sequence_start
     rng = np.random.default_rng(3)
     for n in range(9):
