@@ -214,8 +214,9 @@ extern "C" int32_t qdc_linear_f32(float *out, float *residual, const float *a, c
     if (row_tiles > 65535) return QDC_ERR_SHAPE;
     if (!out || !a || !w || (input != 0 && (!b || !norm)) || (input == 1 && !residual))
         return QDC_ERR_NULL;
-    if (!aligned16(out) || !aligned16(a) || !aligned16(w) || !aligned16(b) || !aligned16(norm) ||
-        !aligned16(residual) || ((uintptr_t)mask & 3u))
+    if (!aligned16(out) || !aligned16(a) || !aligned16(w) ||
+        (input != 0 && (!aligned16(b) || !aligned16(norm))) ||
+        (input == 1 && (!aligned16(residual) || ((uintptr_t)mask & 3u))))
         return QDC_ERR_SHAPE;
     const int64_t out_bytes = ((rows - 1) * ld_out + cols) * 4, res_bytes = rows * inner * 4;
     const int64_t a_bytes = ((rows - 1) * ld_a + inner) * 4, b_bytes = ((rows - 1) * ld_b + inner) * 4;

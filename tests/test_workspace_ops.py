@@ -493,6 +493,18 @@ def test_linear_f32_validation():
     assert f(rows=0, out=None) == 0
 
 
+def test_linear_f32_ignores_unused_pointers():
+    """Pointers an input does not use are ignored, wherever they point: the calls get as
+    far as the overlap of out and a (-5)."""
+    lib = _lib.lib()
+    odd = BIG + 1
+    for inp, res, b, norm, mask in ((0, odd, odd, odd, odd), (2, odd, BIG, BIG, odd)):
+        assert lib.qdc_linear_f32(FAKE, res, FAKE + 16, b, norm, mask, BIG, 5, 256, 128, 128, 256, 256,
+                                  256, 128, 1e-6, inp, 0, None) == -5, inp
+    assert lib.qdc_linear_f32(FAKE, FAKE + (1 << 30), FAKE + 16, BIG, BIG, odd, BIG, 5, 256, 128, 128,
+                              256, 256, 256, 128, 1e-6, 1, 0, None) == -2
+
+
 LINEAR_F32 = [(1, 128, 64), (15, 256, 128), (16, 512, 64), (17, 256, 1792), (64, 512, 256),
               (129, 128, 192), (411, 256, 512)]
 
