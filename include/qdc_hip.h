@@ -71,9 +71,10 @@ typedef enum {
  * qdc_swiglu take out_dtype before the stream; 0.3.0: qdc_delta_prologue and
  * qdc_delta_scan take the q/k and v row strides ld_qk, ld_v before the
  * stream), the patch number with added entry points (0.2.1: qdc_row_scale,
- * qdc_row_scale_check; 0.3.1: qdc_copy_pair).
+ * qdc_row_scale_check; 0.3.1: qdc_copy_pair; 0.3.2: those of
+ * qdc_hip_workspace.h).
  */
-#define QDC_HIP_VERSION "qdc_hip 0.3.1"
+#define QDC_HIP_VERSION "qdc_hip 0.3.2"
 
 /* Library version string ("qdc_hip <major>.<minor>.<patch>"), QDC_HIP_VERSION. */
 const char *qdc_version(void);

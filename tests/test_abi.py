@@ -40,10 +40,11 @@ def test_version_matches_the_header():
     """qdc_version() is the QDC_HIP_VERSION of the header the library was built
     from (0.2.0: out_dtype added to qdc_gated_rmsnorm and qdc_swiglu; 0.2.1:
     qdc_row_scale and qdc_row_scale_check added; 0.3.0: q/k and v row strides
-    added to qdc_delta_prologue and qdc_delta_scan; 0.3.1: qdc_copy_pair added)."""
+    added to qdc_delta_prologue and qdc_delta_scan; 0.3.1: qdc_copy_pair added;
+    0.3.2: the entry points of qdc_hip_workspace.h added)."""
     m = re.search(r'#define\s+QDC_HIP_VERSION\s+"([^"]+)"', open(HEADER).read())
     assert m and re.fullmatch(r"qdc_hip \d+\.\d+\.\d+", m.group(1))
-    assert _lib.version() == m.group(1) == "qdc_hip 0.3.1"
+    assert _lib.version() == m.group(1) == "qdc_hip 0.3.2"
 
 
 def test_status_strings():
