@@ -46,7 +46,7 @@ struct Attention {
     const void *q, *k, *v, *gate;
     const int32_t *mask;  // [batch, S] or null
     int64_t q_tok, q_head, k_tok, k_head, v_tok, v_head, gate_tok, gate_head, out_tok;
-    int S, H, KV, G;
+    int S, KV, G;
     int units;            // G * query blocks, per KV head
     float scale_log2;     // scale * log2(e)
 };
@@ -600,7 +600,6 @@ extern "C" int32_t qdc_attention_fused(void *out, int32_t out_dtype, const void 
     a.gate_head = gate_head;
     a.out_tok = out_tok;
     a.S = (int)seq;
-    a.H = (int)heads;
     a.KV = (int)kv_heads;
     a.G = (int)(heads / kv_heads);
     a.units = (int)units;

@@ -57,7 +57,7 @@ struct ChunkArgs {
     const float *q, *k, *v, *beta, *decay;
     float *ws;
     int64_t ld_qk, ld_v;  // elements between the token rows of q and k, and of v
-    int S, H, KH, vd, groups, chunks, slices;  // slices = vd / 16
+    int S, H, vd, groups, chunks, slices;  // slices = vd / 16
     int64_t units;        // batch * heads * chunks (prepare)
     FastDiv by_chunks, by_heads, by_groups;  // by_groups: workgroups per head (scan)
 };
@@ -578,7 +578,6 @@ extern "C" int32_t qdc_delta_scan_ws(void *out, int32_t out_dtype, const float *
     a.ld_v = ld_v;
     a.S = (int)seq;
     a.H = (int)heads;
-    a.KH = (int)key_heads;
     a.vd = (int)value_dim;
     a.groups = (int)(heads / key_heads);
     a.chunks = (int)ceil_div(seq, (int64_t)kC);

@@ -21,11 +21,11 @@ before a DeltaNet layer, with its input mask (``qdc_residual_rmsnorm_masked``),
 post-attention residual + RMSNorm, the attention prologue (q/k norm + partial
 RoPE, read straight out of the packed projection), causal attention with its
 masked softmax and output gate in one pass over the heads, the DeltaNet prologue
-(convolution, SiLU, q/k L2 norm, gates), the gated-delta recurrence, the DeltaNet gated RMSNorm reading z inside the packed projection,
-and SwiGLU reading the packed gate||up GEMM output.  GEMMs run through
-PyTorch-ROCm (hipBLASLt), with fp32 results; attention scores, exponentials and
-their sums are fp32 (the exponentials enter the product with V in the model
-dtype).  Head sizes the attention kernel does not take, and the last-token
+(convolution, SiLU, q/k L2 norm, gates), the gated-delta recurrence, the
+DeltaNet gated RMSNorm reading z inside the packed projection, and SwiGLU
+reading the packed gate||up GEMM output.  GEMMs run through PyTorch-ROCm
+(hipBLASLt), with fp32 results; attention scores, exponentials and their sums
+are fp32 (the exponentials enter the product with V in the model dtype).  Head sizes the attention kernel does not take, and the last-token
 forward's single query per head, run the two attention products as batched GEMMs
 around the softmax and gate kernels.
 
@@ -347,9 +347,6 @@ class QwenBackbone:
         return ops.native_residual_rms(h, self._mm32(a, layer[name]), norm, self.cfg.eps,
                                        token_mask=token_mask, out_dtype=out_dtype)
 
-    def _full_attention(self, layer, x, mask32, B, S):
-        return self._mm32(self._attention_context(layer, x, mask32, B, S), layer["out"])
-
     def _attention_context(self, layer, x, mask32, B, S):
         """What the output projection of a full-attention layer multiplies:
         ``full_attention`` in the AMDGPU form (``ext/amdgpu_attention.jl:108-178``;
@@ -431,9 +428,6 @@ class QwenBackbone:
         if a.dtype == torch.float32:
             return torch.bmm(a, b)
         return torch.bmm(a, b, out_dtype=torch.float32)
-
-    def _delta_attention(self, layer, x, B, S):
-        return self._mm32(self._delta_context(layer, x, B, S), layer["out"])
 
     def _delta_context(self, layer, x, B, S):
         """What the output projection of a DeltaNet layer multiplies: gated

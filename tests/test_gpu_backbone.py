@@ -453,8 +453,7 @@ def _teacher_forced_layer(model, cfg, i, tr, h, normed, mask):
         gated = ops.native_gated_rms(g(tr["result"], bf).view(T, vh, vd),
                                      proj[:, cq:cq + vw].view(T, vh, vd), L["norm"], eps)
         out.append(("gated RMSNorm", c(gated), tr["gated"], "fused"))
-        out.append(("DeltaNet block", c(model._delta_attention(L, g(tr["masked"], bf), 1, T)),
-                    tr["mixed"], "block"))
+        context = model._delta_context(L, g(tr["masked"], bf), 1, T)
     else:
         hd, H, KV = cfg.head_dim, cfg.heads, cfg.kv_heads
         q, k = ops.prepare_heads(g(tr["qgate"], bf)[:, :, :hd], g(tr["k_proj"], bf), L["q_norm"],
@@ -467,8 +466,11 @@ def _teacher_forced_layer(model, cfg, i, tr, h, normed, mask):
         merged = ops.attention_gate(g(tr["values"]).view(1, H, T, hd),
                                     g(tr["qgate"], bf)[:, :, hd:], out_dtype=bf)
         out.append(("attention gate merge", c(merged), tr["merged"], "fused"))
-        out.append(("attention block", c(model._full_attention(L, g(normed, bf), mask32, 1, T)),
-                    tr["mixed"], "block"))
+        context = model._attention_context(L, g(normed, bf), mask32, 1, T)
+    # the output projection the forward takes at this size, added to nothing
+    mixed, _ = model._project_add_norm(torch.zeros_like(g(h)), context, L, "out", L["post_norm"])
+    out.append(("DeltaNet block" if cfg.layer_types[i] == "linear_attention" else "attention block",
+                c(mixed), tr["mixed"], "block"))
     residual, post = ops.native_residual_rms(g(h), g(tr["mixed"]), L["post_norm"], eps)
     out += [("post-attention residual", c(residual), tr["residual"], "f32"),
             ("post-attention RMSNorm", c(post), tr["post_normed"], "fused")]
@@ -488,16 +490,16 @@ def _free_running_layer(model, cfg, i, h, normed, mask):
     L = model.layers[i]
     mask32 = torch.from_numpy(mask.astype(np.int32)).to(model.device).view(1, -1)
     if cfg.layer_types[i] == "full_attention":
-        mixed = model._full_attention(L, normed, mask32, 1, T)
+        context = model._attention_context(L, normed, mask32, 1, T)
     else:  # the forward's masked norm writes 0/1 times the row: the same values
-        mixed = model._delta_attention(L, normed * mask32.view(-1, 1).to(normed.dtype), 1, T)
-    residual, post = ops.native_residual_rms(h, mixed, L["post_norm"], cfg.eps)
+        context = model._delta_context(L, normed * mask32.view(-1, 1).to(normed.dtype), 1, T)
+    residual, post = model._project_add_norm(h, context, L, "out", L["post_norm"])
     gate_up = post @ L["gate_up"]
     inter = gate_up.shape[1] // 2
     act = ops.native_mlp_gate(gate_up[:, :inter], gate_up[:, inter:])
     last = i + 1 == len(cfg.layer_types)
     nxt = model.final_norm if last else model.layers[i + 1]["input_norm"]
-    return ops.native_residual_rms(residual, model._mm32(act, L["down"]), nxt, cfg.eps)
+    return model._project_add_norm(residual, act, L, "down", nxt)
 
 
 @pytest.mark.timeout(900)
