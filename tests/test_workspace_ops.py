@@ -293,6 +293,69 @@ def test_attention_fused_scales(B, S, H, KV, hd, kind, dtype, scale):
     assert ((got - exact).abs() <= bound).all(), ((got - exact).abs() / bound).max()
 
 
+def rescalings(scores, dtype):
+    """Walks the kernel's order over scaled scores ``[B, H, S, S]`` (-inf: not seen): 32
+    queries a wavefront, keys in steps of 64 (bf16) or tiles of 32 dealt to four
+    wavefronts (fp32); where a lane's maximum passes what its exponents are taken from by
+    2^8, all queries of the wavefront move to their own.  Returns how often that happens to
+    sums that are not empty, and how often to some of a wavefront's queries only."""
+    x = np.asarray(scores) * np.log2(np.e)
+    S = x.shape[-1]
+    tile, walks = (64, 1) if dtype == torch.bfloat16 else (32, 4)
+    half = np.arange(S) % 8 // 4  # which half-wavefront holds a key
+    full = partly = 0
+    for rows in x.reshape(-1, S, S):
+        for q0 in range(0, S, 32):
+            block = rows[q0:q0 + 32, :q0 + 32]
+            for w in range(walks):
+                base = np.full(block.shape[0], -np.inf)
+                for k0 in range(w * tile, block.shape[1], walks * tile):
+                    part = block[:, k0:k0 + tile]
+                    h = half[k0:k0 + part.shape[1]]
+                    tops = np.stack([part[:, h == n].max(1, initial=-np.inf) for n in (0, 1)], 1)
+                    seen = tops > -np.inf
+                    if (seen & (tops > base[:, None] + 8)).any():
+                        moved = tops.max(1) > base
+                        held = np.isfinite(base)
+                        full += (moved & held).any()
+                        partly += (moved & held).any() and (~moved & held).any()
+                        base = np.maximum(base, tops.max(1))
+    return full, partly
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("B,S,H,KV,hd,holes", [(1, 420, 4, 2, 64, False), (2, 450, 3, 1, 128, True),
+                                               (1, 500, 4, 1, 256, True)])
+def test_attention_fused_rescales(B, S, H, KV, hd, holes, dtype):
+    """Scores that rise by 6 to 12 every 96 keys for half of the queries and stay level
+    for the others, so that sums already begun are rescaled, in some lanes only, again and
+    again.  Scores reach 60: a product's error of up to (hd / 2) roundings of its terms'
+    sum moves a weight by that much, twice (its own and the maximum's); otherwise the
+    bounds of the edges."""
+    from qdc_amd import ops
+    rng = np.random.default_rng(S + hd)
+    T, scale = B * S, hd ** -0.5
+    q, k, v, gate = (rng.standard_normal((T, n, hd), dtype=np.float32) for n in (H, KV, KV, H))
+    q[..., 0] = hd ** 0.25 * rng.uniform(0.5, 1.0, (T, H)) * (rng.random((T, H)) < 0.5)
+    k[..., 0] = hd ** 0.25 * (12.0 * (np.arange(T) % S // 96))[:, None]
+    q, k, v, gate = (torch.from_numpy(x).to(dtype).cuda() for x in (q, k, v, gate))
+    mask = None
+    if holes:
+        mask = torch.from_numpy((rng.random((B, S)) < 0.7).astype(np.int32)).cuda()
+    exact, spread, scores = attention_exact(q, k, v, gate, mask, scale, B)
+    full, partly = rescalings(scores, dtype)
+    assert full > 20 and partly > 20
+    size = [x.double().cpu().abs() for x in (q, k)]
+    terms = max((size[0][:, h] @ size[1][:, h // (H // KV)].t()).max().item() for h in range(H)) * scale
+    bound = spread * (1e-5 + 2 * hd / 2 * 2.0 ** -24 * terms
+                      + (2.0 ** -8 if dtype == torch.bfloat16 else 0.0)) + 1e-30
+    got = ops.attention_fused(q, k, v, gate, mask, scale, B, out_dtype=torch.float32)
+    got = got.double().cpu().view(B, S, H, hd)
+    assert torch.isfinite(got).all()
+    assert ((got - exact).abs() <= bound).all(), ((got - exact).abs() / bound).max()
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("out", ["f32", "bf16", "split"])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
