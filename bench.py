@@ -293,8 +293,9 @@ def build_forward_kernels(dev):
     """The fused row kernels exactly as one bf16 forward of the 0.8B-like
     backbone launches them (8 x 2048 = 16384 tokens; fp32 residual stream, bf16
     GEMM activations, q/k read in place from the packed projection and written
-    head-major per sequence, z read in place from the DeltaNet projection),
-    each over rotating buffer sets like the per-kernel benchmark."""
+    token-major, z read in place from the DeltaNet projection), each over rotating
+    buffer sets like the per-kernel benchmark.  Group "standalone": launches at the
+    same shapes that the forward has replaced."""
     import torch
     from qdc_amd import ops
     from qdc_amd.config import qwen35_08b_config
@@ -356,6 +357,18 @@ def build_forward_kernels(dev):
     tables = ops.rope_tables(S, rd, cfg.rope_theta, dev)
     qkv_w = 2 * hd * nh + 2 * hd * kv
 
+    def heads_launch(s):  # what the attention kernel reads
+        ops.prepare_heads(s[0][:, :hd * nh].view(T, nh, hd),
+                          s[0][:, hd * nh:hd * (nh + kv)].view(T, kv, hd), qn, kn, tables, rd, 1e-6,
+                          seq_len=S, q_out=s[1], k_out=s[2])
+    ks.append(Kernel(
+        "fwd_qk_norm_rope_bf16", "qk_norm_rope_fast",
+        2 * T * (nh + kv) * hd * 2 + 2 * hd * 2 + 2 * S * (rd // 2) * 4,
+        lambda i: (randn((T, qkv_w), bf), torch.empty((T, nh, hd), dtype=bf, device=dev),
+                   torch.empty((T, kv, hd), dtype=bf, device=dev)),
+        heads_launch, [T, nh, kv, hd, rd], "bfloat16", group="forward", launches=n_full))
+
+    # the prologue of the form with a score matrix (other head sizes)
     def prep_launch(s):  # the packed projection [q | k | v | gate] as the forward lays it out
         ops.attention_prepare(s[0][:, :hd * nh].view(T, nh, hd),
                               s[0][:, hd * nh:hd * (nh + kv)].view(T, kv, hd),
@@ -367,7 +380,7 @@ def build_forward_kernels(dev):
         lambda i: (randn((T, qkv_w), bf), torch.empty((B, nh, S, hd), dtype=bf, device=dev),
                    torch.empty((B, kv, hd, S), dtype=bf, device=dev),
                    torch.empty((B, kv, S, hd), dtype=bf, device=dev)),
-        prep_launch, [B, S, nh, kv, hd, rd], "bfloat16", group="forward", launches=n_full))
+        prep_launch, [B, S, nh, kv, hd, rd], "bfloat16", group="standalone"))
     vh, vd = cfg.value_heads, cfg.value_dim
     cq = 2 * cfg.key_dim * cfg.key_heads + vh * vd
     pw = -(-(cq + vh * vd + 2 * vh) // 256) * 256
@@ -412,13 +425,13 @@ def build_forward_kernels(dev):
         lambda s: ops.native_gated_rms(s[0], s[1][:, cq:cq + vh * vd].view(T, vh, vd), wg, 1e-6,
                                        out=s[2], out_dtype=X2),
         [T, vh, vd], "bfloat16->bf16x2", group="split", launches=n_delta))
-    ks.append(Kernel(
+    ks.append(Kernel(  # in the attention kernel at this head size
         "fwd_gate_merge_split", "gate_merge_fast", T * nh * hd * (4 + 2 + 4),
         lambda i: (randn((B, nh, S, hd), f32), randn((T, qkv_w), bf),
                    torch.empty((T, 2 * nh * hd), dtype=bf, device=dev)),
         lambda s: ops.attention_gate(s[0], s[1][:, hd * (nh + 2 * kv):].view(T, nh, hd),
                                      out_dtype=X2, out=s[2]),
-        [B, S, nh, hd], "float32,bfloat16->bf16x2", group="split", launches=n_full))
+        [B, S, nh, hd], "float32,bfloat16->bf16x2", group="standalone"))
     ks.append(Kernel(
         "fwd_swiglu_f32_split", "swiglu_fast", T * I * (4 + 4 + 4),
         lambda i: (randn((T, 2 * I), f32), torch.empty((T, 2 * I), dtype=bf, device=dev)),
@@ -1207,8 +1220,8 @@ captured in a HIP graph, rotating buffer sets > 640 MB per kernel). The rows fol
 timed order: the fused row kernels at their per-kernel benchmark shapes, the widened kernels
 (attention softmax and gate merge, DeltaNet prologue and recurrence), then the `fwd_*` rows, the
 fused row kernels exactly as one forward of the 0.8B-like backbone launches them (8 x 2048 tokens;
-"per fwd" = launches per forward), the two launches `fwd_gather_rms_bf16` fuses, at the same shapes
-(not launched by the forward), and the split-output kernels of the split-GEMM-input forward.
+"per fwd" = launches per forward), launches at the same shapes that the forward has replaced (no
+"per fwd"), and the split-output kernels of the split-GEMM-input forward.
 
 Commands (run from `/tmp` with `TMPDIR=/tmp`, `$R` = repository root), commit {commit}; each
 bench run's stdout and stderr saved beside its rocprofv3 directory, then
@@ -1647,8 +1660,10 @@ def main():
             "pct_peak_forward_weighted": round(100 * fb / fs / 1e9 / PEAK_GBS, 1)}
         if alone:
             line["forward_shapes"]["standalone"] = {
-                "note": "the gather and the first input norm as two launches at the forward's "
-                        "shapes; the forward runs them fused (fwd_gather_rms_bf16)",
+                "note": "launches at the forward's shapes that it has replaced: the gather and the "
+                        "first input norm (fused, fwd_gather_rms_bf16), and the attention "
+                        "prologue and split gate merge of the form with a score matrix (other "
+                        "head sizes)",
                 "kernels": {k.name: entry(k) for k in alone}}
     if split:
         sb = sum(k.launches * k.algo_bytes for k in split)
