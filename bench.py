@@ -1075,8 +1075,24 @@ def traffic_source():
 
 
 # ------------------------------------------------- profile summaries ------
+def _one_launch(disp):
+    """Dispatches with the recurrence's two launches as one: its chunk preparation and
+    the scan that follows, under the scan's signature, their times and counts added."""
+    out, due = [], None
+    for sig, dur, val in disp:
+        if "delta_chunk_prepare" in sig[0]:
+            due = (dur, val)
+            continue
+        if due is not None and "delta_chunk_scan" in sig[0]:
+            dur, val = dur + due[0], None if val is None else val + due[1]
+        due = None
+        out.append((sig, dur, val))
+    return out
+
+
 def _dispatches(path, counter=None):
-    """rocprofv3 CSV rows in dispatch order: (signature, duration us, value)."""
+    """rocprofv3 CSV rows in dispatch order: (signature, duration us, value), one per
+    launch the bench times (:func:`_one_launch`)."""
     import csv
     out = []
     with open(path, newline="") as f:
@@ -1089,7 +1105,7 @@ def _dispatches(path, counter=None):
             val = float(r["Counter_Value"]) if counter is not None else None
             out.append((int(r["Dispatch_Id"]), sig, dur, val))
     out.sort(key=lambda d: d[0])
-    return [d[1:] for d in out]
+    return _one_launch([d[1:] for d in out])
 
 
 def _runs(disp, steps):

@@ -53,3 +53,16 @@ def test_kernel_labels():
     assert bench._kernel_label("Cijk_Ailk_Bljk_SB_MT32x32x64", "GEMM") == \
         "GEMMs (Tensile kernels of the kept library)"
     assert bench._kernel_label("__amd_rocclr_copyBuffer") == "runtime copy"
+
+
+def test_the_scan_counts_as_one_launch():
+    """The recurrence of bench.py's delta_scan is two dispatches a call: folded into one,
+    its graph replays are runs like any other kernel's."""
+    prep, scan = ("void qdc::delta_chunk_prepare<8>(x)", 9, 1), ("void qdc::delta_chunk_scan<8>(x)", 3, 1)
+    steps = 3
+    call = [(prep, 1.0, 10.0), (scan, 4.0, 20.0)]
+    disp = bench._one_launch(_d("x", steps) + call * steps + _d("x", steps) + call * steps)
+    passes, _ = bench._find_passes(bench._runs(disp, steps), ["kx", "scan"], steps)
+    assert passes["scan"][1] == [(scan, 5.0, 30.0)] * steps
+    traced = bench._one_launch([(prep, 1.0, None), (scan, 4.0, None), (("y", 1, 1), 2.0, None)])
+    assert traced == [(scan, 5.0, None), (("y", 1, 1), 2.0, None)]
