@@ -19,12 +19,15 @@
 //
 // What the score matrix cost was memory: at 8 x 2048 tokens, 8 heads over 2 of 256,
 // 1.07 GB of scores written, read and rewritten around the softmax, at odd lengths
-// with unaligned rows.  The two products, softmax and gate merge / this kernel, us:
-// bf16 8 x 2048 800 / 217, 1 x 6001 1340 / 221, 4 x 300 50 / 26; fp32 8 x 2048 2340 /
-// 1374, 1 x 6001 3060 / 1254, 3 x 777 250 / 128.  Bound by the matrix products and
-// what a wavefront issues beside them: bf16 137 GFLOP in 217 us is 630 TFLOP/s, with
-// the loads and LDS writes of a step taken out (timing only) 167 us; fp32 100 TFLOP/s
-// of the 157 of the fp32 matrix cores.
+// with unaligned rows.  Kernel times in a trace that alternates the two, medians, us, the
+// two products, softmax and gate merge / this kernel: bf16 8 x 2048 850 / 298, 1 x 6001
+// 1346 / 266, 4 x 300 48 / 28; fp32 8 x 2048 2480 / 1490, 1 x 6001 3005 / 1310, 3 x 777
+// 227 / 115.  Inside a forward of 8 x 2048 tokens 266 a layer.  Bound by the matrix
+// products and what a wavefront issues beside them: bf16 137 GFLOP in 266 us is 515
+// TFLOP/s, fp32 92 to 100 TFLOP/s of the 157 of the fp32 matrix cores.  The exact sigmoid
+// of the gate, 26 instructions a value in an epilogue that has its SIMD to itself, is
+// 20 to 25 us of the 298 and 4 of the 28; the same bits with a shorter reciprocal were no
+// faster (a branch a value 1034 us a layer, one for eight values 1010, this 987).
 #include <cfloat>
 
 #include "qdc_common.hpp"

@@ -14,19 +14,22 @@
 //
 // Column n of S^T, U and O depends on no other column, so the scan's unit is a
 // slice of 16 value columns: one wavefront runs a whole slice with the state in
-// its accumulators and never meets another wavefront (no LDS, no barrier), or
-// KSPLIT wavefronts share a slice's key rows and add their partial Z and Q S0^T
-// through LDS with one barrier per chunk.
+// its accumulators, or KSPLIT wavefronts share a slice's key rows and add their
+// partial Z and Q S0^T through LDS.  Either way a workgroup meets once a chunk: four
+// whole slices for the k and q rows that they read from LDS together.
 //
-// The fp32 matrix products of the scan (104 of 32 cycles per chunk and slice) bound
-// it when the slices fill the chip, the chain from one chunk's state to the next
-// when they do not.  Both launches, kd = vd = 128, against the one-launch form of
-// qdc_delta_scan.hip, which runs 64 columns in eight wavefronts that meet twice a
-// chunk: 8 x 2048 tokens, 16 heads 319 us (prepare 56) / 420; the same with 32 heads
-// 547 / 836; 2 x 1501, 32 heads 169 / 307; 1 x 777, 16 heads 55 / 161; 1 x 411, 4 heads
-// 32 / 87.  Running addresses of rows and outputs as uniform bases and lane offsets
-// are 27 and 39 us of the first two.  Without the operands' refills (timing only) the scan of 8 x 2048 tokens
-// takes 227 us, so what its loads cost beside the products is the next thing to gain.
+// The fp32 matrix products of the scan (104 of 32 cycles per chunk and slice: 177 us
+// at 2.4 GHz for 128 chunks, a slice a SIMD) bound it when the slices fill the chip,
+// the chain from one chunk's state to the next when they do not.  Kernel times in a
+// trace that alternates the one-launch form of qdc_delta_scan.hip, which runs 64
+// columns in eight wavefronts that meet twice a chunk, with these two, medians, kd =
+// vd = 128, bf16 outputs, us, one launch / scan + prepare: 8 x 2048 tokens, 16 heads
+// 494 / 307 + 57; the same with 32 heads 848 / 479 + 93; 2 x 1501, 32 heads 303 / 147 +
+// 21; 1 x 777, 16 heads 159 / 47 + 6; 1 x 411, 4 heads 85 / 26 + 5.  (Inside a forward
+// of 8 x 2048 tokens 297 + 67.)  Uniform bases and lane offsets for the running
+// addresses of rows and outputs took 27 us off the first and 39 off the second; without
+// the operands' refills (timing only) the scan of the first took 227 us, so what its
+// loads cost beside the products is the next thing to gain.
 #include "qdc_common.hpp"
 #include "qdc_hip_workspace.h"
 
@@ -207,8 +210,9 @@ template <int V> __device__ __forceinline__ void load_vec(const float *p, float 
 }
 
 // One set of operands, each refilled for the next chunk as soon as this one has
-// used it (two or three sets in turn measured no faster).  A wavefront has its SIMD all but to itself, so what is not a matrix product has
-// to issue between them: a group of key blocks' products, then its refill.
+// used it (two or three sets in turn measured no faster).  A wavefront has its SIMD
+// all but to itself, so what is not a matrix product has to issue between them: a
+// group of key blocks' products, then its refill.
 //
 // KSPLIT = 1: the workgroup's four slices are of one head.  Its wavefronts load a
 // chunk's k and q rows once between them, two chunks ahead, into one of two LDS

@@ -20,9 +20,10 @@ attention gate merge) also write the split two-term bf16 form, ``out_dtype=BF16X
 each fp32 result ``v`` as ``hi = bf16(v)`` and ``lo = bf16(v - hi)``, every aligned
 group of 4 elements a 16-byte piece ``[4 hi | 4 lo]``, so a ``[rows, K]`` result
 is a bf16 tensor ``[rows, 2K]``; :func:`split_weight` repeats a GEMM weight's rows
-in the same pattern and :func:`join_split` reads ``hi + lo`` back.  Every call enqueues one kernel of ``libqdc_hip.so`` on the
-tensor device's current PyTorch stream; torch supplies device memory and the
-stream only.  dtype is float32 or bfloat16 (fp32 arithmetic either way).
+in the same pattern and :func:`join_split` reads ``hi + lo`` back.  Every call
+enqueues one kernel of ``libqdc_hip.so`` (:func:`delta_scan` and
+:func:`linear_residual_rms` two) on the tensor device's current PyTorch stream;
+torch supplies device memory and the stream only.  dtype is float32 or bfloat16 (fp32 arithmetic either way).
 Argument errors raise ``ValueError`` before anything is enqueued, as the
 reference raises ``ArgumentError`` / ``DimensionMismatch``: every tensor a call
 reads or writes, caller-supplied outputs included, must be on the device of the
@@ -417,10 +418,12 @@ def linear_residual_rms(x: torch.Tensor, a: torch.Tensor, w: torch.Tensor, weigh
 
 
 def linear_f32_takes(rows: int, inner: int, cols: int) -> bool:
-    """Whether :func:`linear_f32` is the faster form of an fp32 projection
-    ``[rows, inner] x [inner, cols]`` with the row work around it.  Measured up to 512
-    rows, where a forward gains 1.15x (16 rows: 1.20x, the least is 1.07x at 411); every
-    column tile forms its rows again, which costs more the more columns there are."""
+    """Whether :func:`linear_f32` takes an fp32 projection ``[rows, inner] x [inner, cols]``
+    with the row work around it.  Every column tile forms its rows again, which costs more
+    the more rows and columns there are: a decision forward gains 1.24x at 16 rows, 1.19x at
+    64, 1.10x at 128, 1.08x at 411, 1.15x at 512.  512 rows is as far as its error has been
+    measured, not where it stops gaining (513 rows 426 / 352 us, 640 387 / 378, 1024 514 /
+    474, 1536 653 / 628, 3072 1086 / 1052)."""
     return 0 < rows <= 512 and inner in (128, 256, 512) and cols % 64 == 0 and cols <= 2048
 
 
