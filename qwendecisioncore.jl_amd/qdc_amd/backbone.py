@@ -55,7 +55,9 @@ from .weights import read_checkpoint_tensors
 
 
 class QwenBackbone:
-    """A Qwen3.5 hybrid backbone resident on one GPU."""
+    """A Qwen3.5 hybrid backbone resident on one GPU.  The weights are laid out once, at
+    construction, some in two layouts (:meth:`__init__`): other weights are another
+    model, and a tensor in ``layers`` is not to be changed by itself."""
 
     def __init__(self, cfg: BackboneConfig, weights: dict, device="cuda:0",
                  dtype: torch.dtype = torch.float32, split_gemm_inputs: bool | str = False):
@@ -63,7 +65,9 @@ class QwenBackbone:
         residual stream and the returned hidden states are fp32 either way.
         ``split_gemm_inputs`` (bfloat16 only: False, True / ``"all"``, or
         ``"mlp"``) selects the split GEMM inputs described in the module
-        docstring."""
+        docstring.  A bfloat16 model holds a projection into the residual stream
+        twice, transposed and as the checkpoint has it, where some number of rows
+        takes the product cut into parts (``ops.linear_parts_fits``)."""
         if dtype not in (torch.float32, torch.bfloat16):
             raise ValueError("dtype must be float32 or bfloat16")
         modes = {False: None, None: None, "none": None, True: "all", "all": "all", "mlp": "mlp"}
